@@ -23,13 +23,17 @@ ROCM = os.environ.get("ROCM_PATH", "/opt/rocm")
 HIPCC = os.path.join(ROCM, "bin", "hipcc")
 ARCH = os.environ.get("ASSIST_AMD_ARCH", "gfx950")
 
-HIP_SOURCES = ["kernels.hip", "mlp.hip"]
+HIP_SOURCES = ["kernels.hip", "row_kernel.hip", "mlp.hip"]
 CPP_SOURCES = ["spk.cpp", "ascii.cpp", "assist_api.cpp", "batch.cpp"]
-HEADERS = ["device_types.h", "force_model.h", "ias15_tables.h", "kernels.h", "internal.h"]
+HEADERS = ["device_types.h", "force_model.h", "force_terms64.h", "ias15_device.h", "ias15_tables.h", "kernels.h", "internal.h"]
 
 HIP_FLAGS = ["--offload-arch=" + ARCH, "-O3", "-std=c++17", "-fPIC",
              "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",
              "-Wno-unused-command-line-argument"]
+# Flags of single sources.  row_kernel.hip: the machine-level loop-invariant code motion would keep
+# literals and addresses of rarely run code (powers, step ends) in some 40 registers across the kernel's
+# loop, which spills the two waves per SIMD that its registers otherwise allow.
+SOURCE_FLAGS = {"row_kernel.hip": ["-mllvm", "-disable-machine-licm"]}
 CPP_FLAGS = ["-O2", "-std=c++17", "-fPIC", "-D__HIP_PLATFORM_AMD__", "-I" + os.path.join(ROCM, "include"),
              "-Wall", "-Wno-unused-function"]
 
@@ -59,7 +63,7 @@ def build(verbose=False):
     jobs = []
     for f in HIP_SOURCES:
         o = os.path.join(OBJ, f + ".o")
-        jobs.append([HIPCC] + HIP_FLAGS + ["-c", os.path.join(CSRC, f), "-o", o])
+        jobs.append([HIPCC] + HIP_FLAGS + SOURCE_FLAGS.get(f, []) + ["-c", os.path.join(CSRC, f), "-o", o])
     for f in CPP_SOURCES:
         o = os.path.join(OBJ, f + ".o")
         jobs.append(["g++"] + CPP_FLAGS + ["-c", os.path.join(CSRC, f), "-o", o])

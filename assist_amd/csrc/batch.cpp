@@ -6,6 +6,7 @@
 #include <stdlib.h>
 #include <string.h>
 
+#include <algorithm>
 #include <map>
 #include <mutex>
 #include <tuple>
@@ -349,10 +350,9 @@ int lanes_for(int nvec, int requested) {
         return requested;
     }
     if (g > 8) return -1;
-    // default: 8-lane groups for every vector count (they spread the 28 ephemeris targets over 8
-    // lanes and keep the substep cache; 2- and 4-lane groups, which keep 7-14 slots per lane in
-    // registers, were slower in every measured configuration); the autotuner may pick 1 lane for
-    // large real-only batches
+    // default of the group kernels: 8 lanes for every vector count (they spread the 28 ephemeris
+    // targets over 8 lanes and keep the substep cache; 2- and 4-lane groups, which keep 7-14 slots per
+    // lane in registers, were slower in every measured configuration)
     return 8;
 }
 
@@ -520,18 +520,54 @@ namespace {
 std::mutex g_launch_mutex;
 
 struct LaunchShape {
-    int G = 8;         // lanes per system
+    int G = 8;         // lanes per system: 1, 2, 4 or 8 (ias15_kernel) or kRowLanes (ias15_row_kernel)
     int threads = 256; // block size
     int waves = 1;     // kernel variant (register budget for 1 or 2 waves per SIMD)
 };
 
-constexpr int kTuneMinSystems = 16384;  // smaller batches take the default shape
-// Systems per trial launch: many resident rounds even at one lane per system (65,536 lanes fill
-// the GPU), so that every shape is timed at throughput rather than by its slowest systems; with
-// a learned first step a system covers the trial span in a few steps, and 4 systems per lane
-// made the one-lane kernel look slower than 8-lane groups while it is 1.5x faster in full.
+// Batches of this size or more hand out their systems in the queue order.
+constexpr int kOrderMinSystems = 16384;
+// Real-only batches of this size or more choose between 16 lanes and one lane per system by trial
+// launches; everything else takes 16 lanes.  One lane per system needs 65,536 systems to give every
+// SIMD one wave and integrates them at the pace of the slowest lane of each wave: 65,536 systems x 365 d
+// take 54.8 ms on it against 18.9 ms on 16 lanes (mixed form), 131,072 67.5 against 37.1 ms, 262,144
+// 65.1 against 73.8 ms, 1,048,576 227 against 294 ms.
+constexpr int kTuneMinSystems = 131072;
+// Systems per trial launch: many resident rounds even at one lane per system, so that every shape is
+// timed at throughput rather than by its slowest systems.
 constexpr int kTuneSample = 1048576;
 constexpr double kTuneSpan = 30.0;      // days integrated per trial system
+
+// The shape of the 16-lane kernel for n systems.  A trip of a wave takes as long with one system as
+// with four, so systems go one to a wave while every SIMD has room for another wave (blocks of one
+// wave, which spread over the CUs), then up to four to a wave (one block of four waves per CU), and
+// only then does a second wave per SIMD pay (blocks of three waves, two per CU, all that the
+// ephemeris tables in LDS leave room for): 4,096 systems x 7 vectors over 3,650 days take 37.4 ms with
+// one wave per SIMD and 45.0 ms with blocks of three waves, 262,144 over 365 days 152 against 118.7 ms.
+LaunchShape row_shape(int n) {
+    int dev = 0, ncu = 0;
+    if (hipGetDevice(&dev) != hipSuccess ||
+        hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess)
+        ncu = 256;
+    LaunchShape sh;
+    sh.G = kRowLanes;
+    sh.waves = 1;
+    const long long simds = 4LL * ncu;
+    sh.threads = n <= simds ? 64 : (n <= 4 * simds ? 256 : 192);
+    return sh;
+}
+
+// The integration kernel of a launch shape.
+hipError_t launch_shape(const IntegrateArgs& a, bool mixed, const LaunchShape& sh, int blocks, hipStream_t s,
+                        bool set_attributes = true) {
+    if (sh.G == kRowLanes) return launch_ias15_row(a, mixed, blocks, sh.threads, s, set_attributes);
+    return launch_ias15(a, sh.G, mixed, sh.waves, blocks, sh.threads, s, set_attributes);
+}
+
+hipError_t shape_occupancy(const IntegrateArgs& a, bool mixed, const LaunchShape& sh, int* blocks_per_cu) {
+    if (sh.G == kRowLanes) return ias15_row_occupancy(a, mixed, sh.threads, blocks_per_cu);
+    return ias15_occupancy(sh.G, mixed, sh.waves, ext_model(a.fo), ias15_snap(a), a.nvec, sh.threads, blocks_per_cu);
+}
 
 // Replays (capturing it first when new) the launch set_counter + ias15_kernel for `a` on the
 // library's graph stream, after the work already queued on `s`; *ms is the graph's HIP-event time.
@@ -558,7 +594,7 @@ int run_ias15_graph(const IntegrateArgs& a, bool mixed, const LaunchShape& sh, i
         if (!hip_ok(hipStreamBeginCapture(gs, hipStreamCaptureModeThreadLocal), "hipStreamBeginCapture"))
             return ASSIST_BATCH_ERROR_DEVICE;
         const bool launched = hip_ok(launch_set_counter(g_ws.queue, total_groups, gs), "launch(set_counter)") &&
-                              hip_ok(launch_ias15(a, sh.G, mixed, sh.waves, blocks, sh.threads, gs, false), "launch(ias15)");
+                              hip_ok(launch_shape(a, mixed, sh, blocks, gs, false), "launch(ias15)");
         const bool captured = hip_ok(hipStreamEndCapture(gs, &graph), "hipStreamEndCapture");
         if (!launched || !captured || !hip_ok(hipGraphInstantiate(&exec, graph, nullptr, nullptr, 0), "hipGraphInstantiate")) {
             if (graph) (void)hipGraphDestroy(graph);
@@ -588,9 +624,7 @@ int run_ias15(IntegrateArgs a, bool mixed, const LaunchShape& sh, int blocks_per
     int dev = 0, ncu = 0, per_cu = 0;
     if (!hip_ok(hipGetDevice(&dev), "hipGetDevice") ||
         !hip_ok(hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, dev), "hipDeviceGetAttribute") ||
-        !hip_ok(ias15_occupancy(sh.G, mixed, sh.waves, ext_model(a.fo), ias15_snap(a), a.nvec, sh.threads,
-                                &per_cu),
-                "occupancy"))
+        !hip_ok(shape_occupancy(a, mixed, sh, &per_cu), "occupancy"))
         return ASSIST_BATCH_ERROR_DEVICE;
     if (per_cu < 1) per_cu = 1;
     if (blocks_per_cu_cap > 0 && blocks_per_cu_cap < per_cu) per_cu = blocks_per_cu_cap;
@@ -599,7 +633,12 @@ int run_ias15(IntegrateArgs a, bool mixed, const LaunchShape& sh, int blocks_per
     // 8-lane groups fill the grid even for batches smaller than it: the kernel spreads the systems
     // over every wave, and the groups without one take Chebyshev items of their wave
     const bool spread = ias15_cache_words(sh.G, ext_model(a.fo)) > 0;
-    const int blocks = (int)((need_blocks < max_blocks && !spread) ? need_blocks : max_blocks);
+    int blocks = (int)((need_blocks < max_blocks && !spread) ? need_blocks : max_blocks);
+    if (sh.G == kRowLanes) {
+        // one system per wave while waves are left: the rows without one help in its ephemeris rounds
+        const long long waves = sh.threads / 64;
+        blocks = (int)std::min((a.nsys + waves - 1) / waves, max_blocks);
+    }
     const int total_groups = blocks * sh.threads / sh.G;
     // scratch: the b/e records of every lane (42 doubles), then the substep ephemeris cache
     const int cw = use_cache ? ias15_cache_words(sh.G, ext_model(a.fo)) : 0;
@@ -616,7 +655,7 @@ int run_ias15(IntegrateArgs a, bool mixed, const LaunchShape& sh, int blocks_per
     }
     if (!hip_ok(launch_set_counter(g_ws.queue, total_groups, s), "launch(set_counter)") ||
         !hip_ok(hipEventRecord(g_ws.ev0, s), "hipEventRecord") ||
-        !hip_ok(launch_ias15(a, sh.G, mixed, sh.waves, blocks, sh.threads, s), "launch(ias15)") ||
+        !hip_ok(launch_shape(a, mixed, sh, blocks, s), "launch(ias15)") ||
         !hip_ok(hipEventRecord(g_ws.ev1, s), "hipEventRecord") || !hip_ok(hipEventSynchronize(g_ws.ev1), "ias15"))
         return ASSIST_BATCH_ERROR_DEVICE;
     float t = 0.f;
@@ -627,22 +666,23 @@ int run_ias15(IntegrateArgs a, bool mixed, const LaunchShape& sh, int blocks_per
 }
 
 struct TuneKey {
-    int dev, nvec, mixed, forces, has_params, cache;
+    int dev, size, mixed, forces, has_params;  // size: the systems' power of two
     bool operator<(const TuneKey& o) const {
-        return std::tie(dev, nvec, mixed, forces, has_params, cache) <
-               std::tie(o.dev, o.nvec, o.mixed, o.forces, o.has_params, o.cache);
+        return std::tie(dev, size, mixed, forces, has_params) <
+               std::tie(o.dev, o.size, o.mixed, o.forces, o.has_params);
     }
 };
 std::map<TuneKey, LaunchShape> g_tuned;
 
-// Picks lanes per system, block size and kernel variant for this batch's configuration by
-// timing each candidate on copies of the first kTuneSample systems over at most kTuneSpan days
-// (the caller's buffers are not touched), with the substep cache as the launch will run it; the
-// choice is cached per device and configuration.
-int tuned_shape(const IntegrateArgs& base, bool mixed, bool use_cache, hipStream_t s, LaunchShape* out) {
+// Picks the kernel and block size for a real-only batch by timing each candidate on copies of its
+// first kTuneSample systems over at most kTuneSpan days (the caller's buffers are not touched); the
+// choice is cached per device, configuration and size class.
+int tuned_shape(const IntegrateArgs& base, bool mixed, hipStream_t s, LaunchShape* out) {
     int dev = 0;
     if (!hip_ok(hipGetDevice(&dev), "hipGetDevice")) return ASSIST_BATCH_ERROR_DEVICE;
-    const TuneKey key{dev, base.nvec, mixed ? 1 : 0, base.fo.forces, base.params ? 1 : 0, use_cache ? 1 : 0};
+    int size = 0;
+    while (size < 30 && (base.nsys >> (size + 1)) > 0) size++;
+    const TuneKey key{dev, size, mixed ? 1 : 0, base.fo.forces, base.params ? 1 : 0};
     auto it = g_tuned.find(key);
     if (it != g_tuned.end()) {
         *out = it->second;
@@ -678,35 +718,28 @@ int tuned_shape(const IntegrateArgs& base, bool mixed, bool use_cache, hipStream
     a.archive = nullptr;
     a.archive_count = nullptr;
     a.archive_cap = 0;
+    LaunchShape one;
+    one.G = 1;
+    LaunchShape one_small = one;
+    one_small.threads = 128;
     LaunchShape best;
-    best.G = lanes_for(base.nvec, 0);
     float best_ms = 1e30f;
-    // candidates: one lane per system (real-only systems) and 8-lane groups, 1 wave per SIMD;
-    // 2- and 4-lane groups and the 2-wave variant were slower in every measured configuration
-    // (they stay available through assist_batch_config)
-    for (int G : {1, 8}) {
-        if (G < base.nvec) continue;
-        for (int threads : {256, 128}) {
-            LaunchShape sh;
-            sh.G = G;
-            sh.threads = threads;
-            sh.waves = 1;
-            // each shape runs twice and keeps the faster time: a kernel's first launch can
-            // include loading its code, which the events around it would count
-            float ms = 1e30f;
-            for (int rep = 0; rep < 2; rep++) {
-                if (!hip_ok(hipMemcpyAsync(st.p, base.states, sw * sizeof(double), hipMemcpyDeviceToDevice, s),
-                            "hipMemcpyAsync"))
-                    return ASSIST_BATCH_ERROR_DEVICE;
-                float t_ms = 0.f;
-                const int rc = run_ias15(a, mixed, sh, 0, s, &t_ms, nullptr, false, use_cache);
-                if (rc) return rc;
-                if (t_ms < ms) ms = t_ms;
-            }
-            if (ms < best_ms) {
-                best_ms = ms;
-                best = sh;
-            }
+    for (const LaunchShape& sh : {row_shape(m), one, one_small}) {
+        // each shape runs twice and keeps the faster time: a kernel's first launch can include loading
+        // its code, which the events around it would count
+        float ms = 1e30f;
+        for (int rep = 0; rep < 2; rep++) {
+            if (!hip_ok(hipMemcpyAsync(st.p, base.states, sw * sizeof(double), hipMemcpyDeviceToDevice, s),
+                        "hipMemcpyAsync"))
+                return ASSIST_BATCH_ERROR_DEVICE;
+            float t_ms = 0.f;
+            const int rc = run_ias15(a, mixed, sh, 0, s, &t_ms, nullptr, false, false);
+            if (rc) return rc;
+            if (t_ms < ms) ms = t_ms;
+        }
+        if (ms < best_ms) {
+            best_ms = ms;
+            best = sh;
         }
     }
     g_tuned[key] = best;
@@ -955,18 +988,20 @@ static int integrate_device_locked(const struct assist_ephem* ephem, const struc
     // the extended force model (geocentric, several EIH sources) runs in FP64 with the 1-wave kernel
     const bool ext = ext_model(a.fo);
     if (ext && (mixed || shape.waves != 1)) return ASSIST_BATCH_ERROR_UNSUPPORTED;
-    const bool tune = lanes_req == 0 && cfg.block_size == 0 && cfg.waves_per_simd == 0 &&
-                      n >= kTuneMinSystems && !dense && !ext;
+    // with no launch override: 16 lanes per system, or one (the checkpoint features and the extended
+    // force model run on the group kernels alone)
+    const bool choose = lanes_req == 0 && cfg.block_size == 0 && cfg.waves_per_simd == 0 && !ext && !ias15_snap(a);
+    if (choose) shape = row_shape(n);
     // the substep cache pays when attempts take several passes: by default it is off with the
     // first-pass stop (configuration 4 mixed+learned: 158.3 ms without it, 161.9 ms with it)
     const bool cache = cfg.substep_cache_off < 0 || (cfg.substep_cache_off == 0 && a.io.pc_tol1 <= 0.0);
-    if (tune) {
-        rc = tuned_shape(a, mixed, cache, s, &shape);
+    if (choose && nv == 1 && n >= kTuneMinSystems && !dense) {
+        rc = tuned_shape(a, mixed, s, &shape);
         if (rc) return rc;
     }
     // large batches: hand out the systems of highest expected cost first (longest spans, smallest
     // perihelia), so that the launch does not end on an expensive system handed out last
-    if (n >= kTuneMinSystems && !dense && d_t1 && !a.snap_in) {
+    if (n >= kOrderMinSystems && !dense && d_t1 && !a.snap_in) {
         rc = ensure_workspace(0);
         if (rc) return rc;
         rc = ensure_order(n);
@@ -1021,10 +1056,18 @@ int assist_batch_integrate_device_noalloc(const struct assist_ephem* ephem, cons
     const bool mixed = cfg.precision == ASSIST_PRECISION_MIXED;
     const bool ext = ext_model(a.fo);
     if (ext && mixed) return ASSIST_BATCH_ERROR_UNSUPPORTED;
-    const int G = lanes_for(nv, cfg.lanes_per_system);
-    const int threads = cfg.block_size > 0 ? cfg.block_size : kIas15Block;
-    if (G < 0 || threads % 64 != 0 || threads > kIas15Block || threads % G != 0) return ASSIST_BATCH_ERROR_ARG;
-    if (cfg.waves_per_simd != 0 && cfg.waves_per_simd != 1) return ASSIST_BATCH_ERROR_UNSUPPORTED;
+    LaunchShape shape;
+    if (cfg.lanes_per_system == 0 && cfg.block_size == 0 && cfg.waves_per_simd == 0 && !ext) {
+        shape = row_shape(n);
+    } else {
+        shape.G = lanes_for(nv, cfg.lanes_per_system);
+        shape.threads = cfg.block_size > 0 ? cfg.block_size : kIas15Block;
+        shape.waves = 1;
+        if (shape.G < 0 || shape.threads % 64 != 0 || shape.threads > kIas15Block || shape.threads % shape.G != 0)
+            return ASSIST_BATCH_ERROR_ARG;
+        if (cfg.waves_per_simd != 0 && cfg.waves_per_simd != 1) return ASSIST_BATCH_ERROR_UNSUPPORTED;
+    }
+    const int G = shape.G, threads = shape.threads;
     a.io.epsilon = cfg.epsilon;
     a.io.min_dt = cfg.min_dt;
     a.io.dt_initial = cfg.dt_initial;
@@ -1046,13 +1089,14 @@ int assist_batch_integrate_device_noalloc(const struct assist_ephem* ephem, cons
     int dev = 0, ncu = 0, per_cu = 0;
     if (!hip_ok(noalloc_scratch(&scr), "hipGetSymbolAddress(scratch)") || !hip_ok(hipGetDevice(&dev), "hipGetDevice") ||
         !hip_ok(hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, dev), "hipDeviceGetAttribute") ||
-        !hip_ok(ias15_occupancy(G, mixed, 1, ext, false, nv, threads, &per_cu), "occupancy"))
+        !hip_ok(shape_occupancy(a, mixed, shape, &per_cu), "occupancy"))
         return ASSIST_BATCH_ERROR_DEVICE;
     if (per_cu < 1) per_cu = 1;
     if (cfg.blocks_per_cu > 0 && cfg.blocks_per_cu < per_cu) per_cu = cfg.blocks_per_cu;
     // the grid: one pass of the persistent kernel over at most kNoAllocLanes resident lanes (the
     // b/e records of the static scratch); the work queue hands every system to them
-    long long blocks = ((long long)n * G + threads - 1) / threads;
+    long long blocks = G == kRowLanes ? ((long long)n + threads / 64 - 1) / (threads / 64)
+                                      : ((long long)n * G + threads - 1) / threads;
     if (blocks > (long long)per_cu * ncu) blocks = (long long)per_cu * ncu;
     if (blocks > kNoAllocLanes / threads) blocks = kNoAllocLanes / threads;
     if (blocks < 1) return ASSIST_BATCH_ERROR_ARG;
@@ -1062,7 +1106,7 @@ int assist_batch_integrate_device_noalloc(const struct assist_ephem* ephem, cons
     const int total_groups = (int)blocks * threads / G;
     hipStream_t s = (hipStream_t)stream;
     if (!hip_ok(launch_set_counter(a.queue, total_groups, s), "launch(set_counter)") ||
-        !hip_ok(launch_ias15(a, G, mixed, 1, (int)blocks, threads, s), "launch(ias15)") ||
+        !hip_ok(launch_shape(a, mixed, shape, (int)blocks, s), "launch(ias15)") ||
         !hip_ok(hipStreamSynchronize(s), "ias15"))
         return ASSIST_BATCH_ERROR_DEVICE;
     return ASSIST_SUCCESS;

@@ -505,7 +505,7 @@ AHD void term_earth_J2J4(const DevEphem& E, const D xr[3], const D xe[3], D GM, 
     const TS J3p = TS(E.k_J3) * tir5;            // 5 J3 Re^3 / (2 r^5)
     const TS J3f = TS(3.) - TS(7.) * ct2;
     const TS J4p = TS(E.k_J4) * (tir5 * tir2);   // 5 J4 Re^4 / (8 r^7)
-    const TS J4f = TS(63.) * ct2 * ct2 - TS(42.) * ct2 + TS(3.);
+    const TS J4f = fma(TS(-42.), ct2, TS(63.) * ct2 * ct2) + TS(3.);
     const TS j3x = -tGM * J3p * tir2 * J3f * tdx * tdz;
     const TS j3y = -tGM * J3p * tir2 * J3f * tdy * tdz;
     const TS j3z = -tGM * J3p * (TS(6.) * ct2 - TS(7.) * ct2 * ct2 - TS(0.6));
@@ -848,7 +848,7 @@ AHD void term_gr_simple(const DevEphem& E, const D xr[3], const D vr[3], const D
     const TS B = TS(4.0) * (p[0] * pv[0] + p[1] * pv[1] + p[2] * pv[2]);
     const TS prefac = G / (r * r * r * TS(E.c_squared));
 #pragma unroll
-    for (int c = 0; c < 3; c++) acc[c] += D(prefac * (A * p[c] + B * pv[c]));
+    for (int c = 0; c < 3; c++) acc[c] += D(prefac * fma(B, pv[c], A * p[c]));
     if (!need_jac) return;
     const TS dpdr = TS(-3.0) * prefac / r;
 #pragma unroll
@@ -861,6 +861,12 @@ AHD void term_gr_simple(const DevEphem& E, const D xr[3], const D vr[3], const D
         }
     }
 }
+
+}  // namespace assist_gpu
+
+#include "force_terms64.h"
+
+namespace assist_gpu {
 
 // ---- the full evaluation ---------------------------------------------------------------------
 template <typename D>
@@ -1195,16 +1201,25 @@ AHD void force_eval(const DevEphem& E, const DevSlot* slots, const double* gm, c
     D acc[3] = {D(0.0), D(0.0), D(0.0)};
     jac_zero(J);
     const D GMs = D(E.GM[0]);
-    if ((forces & F_NONGRAV) && ng) term_nongrav<D, TS>(O, xr, vr, sun, sunv, A, need_jac, acc, J);
-    if (forces & F_EARTH_H) term_earth_J2J4<D, TS>(E, xr, earth, D(E.GM[3]), need_jac, acc, J);
-    if (forces & F_SUN_H) term_solar_J2<D, TS>(E, xr, sun, GMs, need_jac, acc, J);
-    if constexpr (Ext) {
-        if (eih) eih_sources<G>(E, O, gm, lane, xr, vr, px, pv, xo, vo, ao, S0, dS0, need_jac, acc, J);
+    if constexpr (std::is_same<TS, double>::value) {
+        if ((forces & F_NONGRAV) && ng) fp64::term_nongrav(O, xr, vr, sun, sunv, A, need_jac, acc, J);
+        if (forces & F_EARTH_H) fp64::term_earth_J2J4(E, xr, earth, E.GM[3], need_jac, acc, J);
+        if (forces & F_SUN_H) fp64::term_solar_J2(E, xr, sun, GMs, need_jac, acc, J);
+        if constexpr (Ext) {
+            if (eih) eih_sources<G>(E, O, gm, lane, xr, vr, px, pv, xo, vo, ao, S0, dS0, need_jac, acc, J);
+        } else {
+            if (eih) fp64::term_eih_sun(E, xr, vr, sun, sunv, GMs, S0, dS0, S1, aj, need_jac, acc, J);
+        }
+        if (forces & F_GR_POTENTIAL) fp64::term_gr_potential(E, xr, sun, GMs, need_jac, acc, J);
+        if (forces & F_GR_SIMPLE) fp64::term_gr_simple(E, xr, vr, sun, sunv, GMs, need_jac, acc, J);
     } else {
+        if ((forces & F_NONGRAV) && ng) term_nongrav<D, TS>(O, xr, vr, sun, sunv, A, need_jac, acc, J);
+        if (forces & F_EARTH_H) term_earth_J2J4<D, TS>(E, xr, earth, D(E.GM[3]), need_jac, acc, J);
+        if (forces & F_SUN_H) term_solar_J2<D, TS>(E, xr, sun, GMs, need_jac, acc, J);
         if (eih) term_eih_sun<D, TS>(E, xr, vr, sun, sunv, GMs, S0, dS0, S1, aj, need_jac, acc, J);
+        if (forces & F_GR_POTENTIAL) term_gr_potential<D, TS>(E, xr, sun, GMs, need_jac, acc, J);
+        if (forces & F_GR_SIMPLE) term_gr_simple<D, TS>(E, xr, vr, sun, sunv, GMs, need_jac, acc, J);
     }
-    if (forces & F_GR_POTENTIAL) term_gr_potential<D, TS>(E, xr, sun, GMs, need_jac, acc, J);
-    if (forces & F_GR_SIMPLE) term_gr_simple<D, TS>(E, xr, vr, sun, sunv, GMs, need_jac, acc, J);
     if (forces & (F_SUN | F_PLANETS | F_ASTEROIDS)) {
 #pragma unroll
         for (int c = 0; c < 3; c++) acc[c] += ad[c] + D(adt[c]);

@@ -22,6 +22,12 @@ __host__ __device__ constexpr int ias15_cols_per_group(int G, int nvec, int wave
 // to 256 words so that the columns keep their LDS bank alignment.
 constexpr int kTabH = 0, kTabPX = 8, kTabPV = 80, kTabRRI = 143, kTabC = 171, kTabW = 192, kTabWords = 256;
 
+// The kernel with 16 lanes (a DPP row) per system: largest block, and words of LDS per wave (for
+// each of its 4 rows a step attempt's ephemeris, kRowTimes x kRowSlice, and 24 Marsden parameters).
+constexpr int kRowLanes = 16, kRowBlock = 256;
+constexpr int kRowTimes = 8, kRowSlice = 88;
+constexpr int kRowWaveWords = 4 * (kRowTimes * kRowSlice + 24);
+
 struct ForcesArgs {
     const DevEphem* E;
     ForceOpts fo;
@@ -123,6 +129,12 @@ hipError_t launch_ias15(const IntegrateArgs& a, int G, bool mixed, int waves, in
                         bool set_attributes = true);
 hipError_t ias15_occupancy(int G, bool mixed, int waves, bool ext, bool snap, int nvec, int threads,
                            int* blocks_per_cu);
+// The 16-lane kernel (row_kernel.hip), for launches without checkpoint features or the extended
+// force model; its scratch is 28 doubles per launched thread at most.
+hipError_t launch_ias15_row(const IntegrateArgs& a, bool mixed, int blocks, int threads, hipStream_t s,
+                            bool set_attributes = true);
+hipError_t ias15_row_occupancy(const IntegrateArgs& a, bool mixed, int threads, int* blocks_per_cu);
+size_t ias15_row_lds_bytes(int threads);
 // Whether a launch uses the checkpoint, pause or step-archive features (kernels without them
 // exist for the hot shapes).
 inline bool ias15_snap(const IntegrateArgs& a) { return a.snap_in || a.snap_out || a.t_pause || a.archive; }

@@ -46,6 +46,7 @@ inline Cnt operator+(Cnt a) { return a; }
 inline CntF operator+(CntF a) { return a; }
 inline CntF operator-(CntF a) { return CntF(-a.v); }
 inline Cnt fma(Cnt a, Cnt b, Cnt c) { g_ops64 += 2; return Cnt(a.v * b.v + c.v); }
+inline CntF fma(CntF a, CntF b, CntF c) { g_ops32 += 2; return CntF(a.v * b.v + c.v); }
 inline Cnt sqrt(Cnt a) { g_ops64++; return Cnt(::sqrt(a.v)); }
 inline CntF sqrt(CntF a) { g_ops32++; return CntF(::sqrtf(a.v)); }
 inline CntF pow(CntF a, CntF b) { g_ops32++; return CntF(::powf(a.v, b.v)); }

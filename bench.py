@@ -59,7 +59,7 @@ def opcounts():
 def algorithmic_flops(oc, nvec, ng, mixed, evals, steps, rejected, cached=False):
     """FP64 and FP32 operations of one launch from per-system eval/step counts; ``ng`` is the
     per-system flag of a non-zero Marsden model, ``rejected`` per-system or total rejections.
-    With ``cached`` (the substep ephemeris cache of 8-lane groups), only the evaluations that
+    With ``cached`` (8 and 16 lanes per system evaluate a substep's ephemeris once per attempt), only the evaluations that
     compute fresh positions (each step's first one and the first iteration of every attempt)
     count the Chebyshev series."""
     form = "mixed" if mixed else "fp64"
@@ -355,7 +355,7 @@ def main():
     # (the device entry points report no rejection total; a rejected attempt's 7 fresh evaluations
     # then count as cached ones, so the count is a lower bound; these workloads reject rarely)
     f64, f32 = algorithmic_flops(oc, nv, ng, main_res["mixed"], main_res["evals"], main_res["steps"], st.rejected,
-                                 cached=st.lanes_per_system == 8)
+                                 cached=st.lanes_per_system >= 8)
     kms = main_res["kernel_ms"]
     ach64 = f64 / (kms * 1e-3) / 1e12
     ach32 = f32 / (kms * 1e-3) / 1e12

@@ -263,10 +263,10 @@ struct assist_batch_config {
     double dt_initial;    /* first trial step in days (default 0.001) */
     long long max_steps;  /* per system (default 10^6) */
     int precision;        /* ASSIST_PRECISION_* */
-    int lanes_per_system; /* 0 = choose (autotuned), else 1, 2, 4 or 8 (>= 1 + n_var) */
+    int lanes_per_system; /* 0 = choose (16, or 1 for large real-only batches), else 1, 2, 4 or 8 (>= 1 + n_var) */
     int block_size;       /* 0 = choose, else a multiple of 64 up to 256 */
     int blocks_per_cu;    /* 0 = occupancy limit */
-    int waves_per_simd;   /* 0 = choose (autotuned), else 1 or 2: the kernel variant's register budget */
+    int waves_per_simd;   /* 0 = choose, else 1 or 2: the kernel variant's register budget */
     int use_graph;        /* 1: launch the integration as a captured HIP graph, captured once per
                              argument set and replayed (the launches of a replay take the same
                              device pointers); 0 (default): direct launches */
