@@ -3,15 +3,12 @@
 // pass and Adam update written here as HIP kernels for gfx950.
 //
 // Network: 16 inputs (10 used) -> 128 -> 128 -> 128 (tanh) -> 32 outputs (22 used).  Weights
-// are kept as an FP32 master copy for the optimizer and a BF16 copy that the forward pass
-// feeds to the matrix cores; every product runs on v_mfma_f32_16x16x16_bf16 (BF16 operands,
-// FP32 accumulation).  Activations and gradients are stored in FP32 and rounded to BF16
-// (nearest even) where they enter a product.
+// are kept as an FP32 master copy for the optimizer and BF16 copies for the matrix cores; every
+// product runs on v_mfma_f32_16x16x16_bf16 (BF16 operands, FP32 accumulation).  Activations and
+// gradients are held in FP32 and rounded to BF16 (nearest even) where they enter a product.
 //
-// GEMM mapping: one wave computes one 16 x 16 tile of C = op(A) op(B) (four waves, four
-// tiles, per workgroup); each MFMA consumes a 16 x 16 slice of the reduction dimension.  For
-// the weight gradients (reduction over the batch) the reduction is split across workgroups
-// (blockIdx.z) and the partial tiles are added with atomics.
+// MFMA 16x16x16 BF16 operand layout (one wave): lane l holds A[l % 16][4 (l / 16) + j] and
+// B[4 (l / 16) + j][l % 16] for j = 0..3, and receives C[4 (l / 16) + j][l % 16].
 #include <hip/hip_runtime.h>
 #include <math.h>
 #include <stdint.h>
@@ -27,139 +24,27 @@ namespace assist_gpu {
 typedef short bf16x4 __attribute__((ext_vector_type(4)));
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 
-// FP32 -> BF16, round to nearest even (NaN kept quiet).
-__host__ __device__ __forceinline__ uint16_t f2bf(float f) {
-    uint32_t u;
-    memcpy(&u, &f, 4);
-    if ((u & 0x7f800000u) == 0x7f800000u) return (uint16_t)((u >> 16) | ((u & 0xffffu) ? 0x40u : 0u));
-    u += 0x7fffu + ((u >> 16) & 1u);
-    return (uint16_t)(u >> 16);
-}
-__host__ __device__ __forceinline__ float bf2f(uint16_t h) {
-    const uint32_t u = (uint32_t)h << 16;
-    float f;
-    memcpy(&f, &u, 4);
-    return f;
-}
+// FP32 -> BF16, round to nearest even (v_cvt_pk_bf16_f32).
+__device__ __forceinline__ uint16_t f2bf(float f) { return __builtin_bit_cast(uint16_t, (__bf16)f); }
 
-template <typename T>
-__device__ __forceinline__ uint16_t load_bf(const T* p, size_t i);
-template <>
-__device__ __forceinline__ uint16_t load_bf<float>(const float* p, size_t i) { return f2bf(p[i]); }
-template <>
-__device__ __forceinline__ uint16_t load_bf<uint16_t>(const uint16_t* p, size_t i) { return p[i]; }
-
-struct GemmArgs {
-    int M, N, K;
-    const void* A;  // element (i, k): TA ? A[k * lda + i] : A[i * lda + k]
-    int lda;
-    const void* B;  // element (k, j): TB ? B[j * ldb + k] : B[k * ldb + j]
-    int ldb;
-    float* C;       // C[i * ldc + j]
-    int ldc;
-    const float* bias;  // [N] added before the activation, or null
-    int act;            // kActNone or kActTanh
-    int atomic;         // add into C with atomics (split reduction) instead of storing
-    int kchunk;         // reduction length per blockIdx.z (a multiple of 16)
-};
-
-enum : int { kActNone = 0, kActTanh = 1 };
-
-// MFMA 16x16x16 BF16 operand layout (one wave): lane l holds A[l % 16][4 (l / 16) + j] and
-// B[4 (l / 16) + j][l % 16] for j = 0..3, and receives C[4 (l / 16) + j][l % 16].
-template <typename TAe, typename TBe, bool TA, bool TB>
-__global__ void __launch_bounds__(256) gemm_bf16_kernel(GemmArgs g) {
-    const int wave = threadIdx.x >> 6;
-    const int lane = threadIdx.x & 63;
-    const int tiles_n = (g.N + 15) >> 4;
-    const int tile = blockIdx.x * 4 + wave;
-    const int tiles_m = (g.M + 15) >> 4;
-    if (tile >= tiles_m * tiles_n) return;  // whole waves exit
-    const int i0 = (tile / tiles_n) << 4;
-    const int j0 = (tile % tiles_n) << 4;
-    const int k_beg = blockIdx.z * g.kchunk;
-    const int k_end = min(g.K, k_beg + g.kchunk);
-    const TAe* A = (const TAe*)g.A;
-    const TBe* B = (const TBe*)g.B;
-    const int r = lane & 15;
-    const int q = (lane >> 4) << 2;
-    f32x4 acc = {0.f, 0.f, 0.f, 0.f};
-    for (int k0 = k_beg; k0 < k_end; k0 += 16) {
-        bf16x4 a, b;
-#pragma unroll
-        for (int j = 0; j < 4; j++) {
-            const int k = k0 + q + j;
-            const int ia = i0 + r, jb = j0 + r;
-            uint16_t av = 0, bv = 0;
-            if (ia < g.M && k < k_end) av = load_bf<TAe>(A, TA ? (size_t)k * g.lda + ia : (size_t)ia * g.lda + k);
-            if (jb < g.N && k < k_end) bv = load_bf<TBe>(B, TB ? (size_t)jb * g.ldb + k : (size_t)k * g.ldb + jb);
-            a[j] = (short)av;
-            b[j] = (short)bv;
-        }
-        acc = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(a, b, acc, 0, 0, 0);
-    }
-    const int jc = j0 + r;
-    if (jc >= g.N) return;
-#pragma unroll
-    for (int j = 0; j < 4; j++) {
-        const int ic = i0 + q + j;
-        if (ic >= g.M) continue;
-        float v = acc[j];
-        if (g.bias) v += g.bias[jc];
-        if (g.act == kActTanh) v = tanhf(v);
-        float* dst = g.C + (size_t)ic * g.ldc + jc;
-        if (g.atomic) atomicAdd(dst, v);
-        else *dst = v;
-    }
+// Parameter layout: layer by layer, W[in][out] row-major, then b[out].  The BF16 copy is kept twice,
+// in this layout (p16, the operand of the backward products, which reduce over the outputs) and with
+// every W transposed to [out][in] (p16t, the operand of the forward products, which reduce over the
+// inputs), so that a lane's four consecutive operand elements are one 8-byte read in either direction.
+constexpr int kIn = ASSIST_MLP_IN, kHid = ASSIST_MLP_HIDDEN, kOut = ASSIST_MLP_OUT;
+constexpr int kOff1 = 0, kOff2 = kOff1 + kIn * kHid + kHid, kOff3 = kOff2 + kHid * kHid + kHid,
+              kOff4 = kOff3 + kHid * kHid + kHid, kNumParams = kOff4 + kHid * kOut + kOut;
+__device__ __forceinline__ int transposed_pos(int i) {
+    const int off = i < kOff2 ? kOff1 : (i < kOff3 ? kOff2 : (i < kOff4 ? kOff3 : kOff4));
+    const int K = i < kOff2 ? kIn : kHid, N = i < kOff4 ? kHid : kOut;
+    const int e = i - off;
+    return e < K * N ? off + (e % N) * K + e / N : i;
 }
 
-// dZ = dH * (1 - H^2) (tanh derivative from its output), in place on dH.
-__global__ void tanh_backward_kernel(float* dH, const float* H, size_t n) {
-    const size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < n) dH[i] *= 1.f - H[i] * H[i];
-}
-
-// Column sums of X[M][N] added into out[N] (bias gradients).
-__global__ void colsum_kernel(const float* X, int M, int N, float* out) {
-    const int j = blockIdx.y;
-    float s = 0.f;
-    for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < M; i += gridDim.x * blockDim.x) s += X[(size_t)i * N + j];
-    for (int m = 32; m >= 1; m >>= 1) s += __shfl_xor(s, m, 64);
-    __shared__ float part[4];
-    if ((threadIdx.x & 63) == 0) part[threadIdx.x >> 6] = s;
-    __syncthreads();
-    if (threadIdx.x == 0) {
-        float t = 0.f;
-        for (int w = 0; w < (int)(blockDim.x >> 6); w++) t += part[w];
-        atomicAdd(out + j, t);
-    }
-}
-
-// Weighted squared error: loss += sum w_j (Y - T)^2 / M, dY = 2 w_j (Y - T) / M.
-__global__ void mse_kernel(const float* Y, const float* T, const float* w, int M, int N, float* dY, float* loss) {
-    const size_t n = (size_t)M * N;
-    float s = 0.f;
-    for (size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (size_t)gridDim.x * blockDim.x) {
-        const int j = (int)(i % N);
-        const float d = Y[i] - T[i];
-        s += w[j] * d * d;
-        dY[i] = 2.f * w[j] * d / (float)M;
-    }
-    for (int m = 32; m >= 1; m >>= 1) s += __shfl_xor(s, m, 64);
-    __shared__ float part[4];
-    if ((threadIdx.x & 63) == 0) part[threadIdx.x >> 6] = s;
-    __syncthreads();
-    if (threadIdx.x == 0) {
-        float t = 0.f;
-        for (int k = 0; k < (int)(blockDim.x >> 6); k++) t += part[k];
-        atomicAdd(loss, t / (float)M);
-    }
-}
-
-// Adam (Kingma & Ba 2015) with bias correction; refreshes the BF16 copy of the weights.
-__global__ void adam_kernel(float* p, uint16_t* p16, const float* g, float* m, float* v, size_t n, float lr, float b1,
-                            float b2, float eps, float c1, float c2) {
-    const size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
+// Adam (Kingma & Ba 2015) with bias correction; refreshes the BF16 copies of the weights.
+__global__ void adam_kernel(float* p, uint16_t* p16, uint16_t* p16t, const float* g, float* m, float* v, int n,
+                            float lr, float b1, float b2, float eps, float c1, float c2) {
+    const int i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= n) return;
     const float gi = g[i];
     const float mi = b1 * m[i] + (1.f - b1) * gi;
@@ -168,42 +53,38 @@ __global__ void adam_kernel(float* p, uint16_t* p16, const float* g, float* m, f
     v[i] = vi;
     const float pi = p[i] - lr * (mi / c1) / (sqrtf(vi / c2) + eps);
     p[i] = pi;
-    p16[i] = f2bf(pi);
+    const uint16_t h = f2bf(pi);
+    p16[i] = h;
+    p16t[transposed_pos(i)] = h;
 }
 
-__global__ void to_bf16_kernel(const float* p, uint16_t* p16, size_t n) {
-    const size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < n) p16[i] = f2bf(p[i]);
-}
-
-__global__ void fill_kernel(float* p, size_t n, float v) {
-    const size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < n) p[i] = v;
+__global__ void to_bf16_kernel(const float* p, uint16_t* p16, uint16_t* p16t, int n) {
+    const int i = blockIdx.x * blockDim.x + threadIdx.x;
+    if (i >= n) return;
+    const uint16_t h = f2bf(p[i]);
+    p16[i] = h;
+    p16t[transposed_pos(i)] = h;
 }
 
 // ---- prediction: the four layers fused in one kernel ----------------------------------------
-// The forward pass for prediction keeps no activations: each wave takes 16 rows at a time
+// The forward pass keeps no activations: each wave takes 16 rows at a time
 // through all four layers, with the BF16 weights staged once per workgroup in LDS (transposed,
 // [out][in], so that a lane's four consecutive inputs of one output are one 8-byte read) and the
 // 16 x 128 activation tile in the wave's own LDS area, through which the MFMA result layout
 // (four rows of one column per lane) becomes the next operand layout (four columns of one row).
-// Every product is the same v_mfma_f32_16x16x16_bf16 over the same 16-wide slices of the
-// reduction in the same order as gemm_bf16_kernel, with the same bias, tanh and BF16 rounding,
-// so the outputs equal assist_mlp_forward's bit for bit.
 // (LDS rows are padded by 4 elements, 8 bytes: the 16 lanes that read one operand slice then
 // fall in distinct banks instead of all in one)
-constexpr int kPIn = ASSIST_MLP_IN, kPH = ASSIST_MLP_HIDDEN, kPOut = ASSIST_MLP_OUT;
 constexpr int kPad = 4;
-constexpr int kPW1 = 0, kPW2 = kPW1 + kPH * (kPIn + kPad), kPW3 = kPW2 + kPH * (kPH + kPad),
-              kPW4 = kPW3 + kPH * (kPH + kPad);
-constexpr int kPWords = kPW4 + kPOut * (kPH + kPad);  // BF16 weights in LDS
-constexpr int kPBias = 3 * kPH + kPOut;                 // FP32 biases in LDS
+constexpr int kPW1 = 0, kPW2 = kPW1 + kHid * (kIn + kPad), kPW3 = kPW2 + kHid * (kHid + kPad),
+              kPW4 = kPW3 + kHid * (kHid + kPad);
+constexpr int kPWords = kPW4 + kOut * (kHid + kPad);  // BF16 weights in LDS
+constexpr int kPBias = 3 * kHid + kOut;                 // FP32 biases in LDS
 constexpr int kPWaves = 16;  // four waves per SIMD share one copy of the weights
-constexpr int kPTileRow = kPH + kPad;
+constexpr int kPTileRow = kHid + kPad;
 constexpr size_t kPLdsBytes = (size_t)kPWords * 2 + (size_t)kPBias * 4 + (size_t)kPWaves * 16 * kPTileRow * 2;
 
 struct PredictArgs {
-    const uint16_t* p16;  // BF16 parameters (layer by layer: W[in][out] row-major, then b[out])
+    const uint16_t* p16t; // BF16 parameters, weights as [out][in]
     const float* p;       // FP32 parameters (the biases are read from here)
     const float* X;       // [M][16]
     float* Y;             // [M][32]
@@ -233,7 +114,7 @@ __device__ __forceinline__ void predict_layer(const bf16x4 (&a)[KC], const uint1
             const float v = acc[j] + bc;
             if constexpr (Last) {
                 const int row = row0 + q + j;
-                if (row < M) Y[(size_t)row * kPOut + col] = v;
+                if (row < M) Y[(size_t)row * kOut + col] = v;
             } else {
                 tile[(q + j) * kPTileRow + col] = f2bf(tanhf(v));
             }
@@ -246,17 +127,17 @@ __global__ void __launch_bounds__(64 * kPWaves) mlp_predict_kernel(PredictArgs g
     uint16_t* const sw = (uint16_t*)s_pred;
     float* const sb = (float*)(s_pred + (size_t)kPWords * 2);
     uint16_t* const tiles = (uint16_t*)(s_pred + (size_t)kPWords * 2 + (size_t)kPBias * 4);
-    // stage the weights transposed ([out][in]) and the biases
+    // stage the weights ([out][in]) and the biases
     {
-        const int dims[5] = {kPIn, kPH, kPH, kPH, kPOut};
+        const int dims[5] = {kIn, kHid, kHid, kHid, kOut};
         const int dst[4] = {kPW1, kPW2, kPW3, kPW4};
         size_t src = 0;
         int boff = 0;
         for (int l = 0; l < 4; l++) {
             const int K = dims[l], N = dims[l + 1];
-            for (int i = threadIdx.x; i < K * N; i += blockDim.x) {
-                const int k = i / N, n = i - k * N;
-                sw[dst[l] + n * (K + kPad) + k] = g.p16[src + i];
+            for (int i = threadIdx.x * 4; i < K * N; i += blockDim.x * 4) {
+                const int n = i / K, k = i - n * K;  // (K is a multiple of 4)
+                *(bf16x4*)(sw + dst[l] + n * (K + kPad) + k) = *(const bf16x4*)(g.p16t + src + i);
             }
             src += (size_t)K * N;
             for (int i = threadIdx.x; i < N; i += blockDim.x) sb[boff + i] = g.p[src + i];
@@ -275,27 +156,328 @@ __global__ void __launch_bounds__(64 * kPWaves) mlp_predict_kernel(PredictArgs g
         {
             const int row = row0 + r;
 #pragma unroll
-            for (int j = 0; j < 4; j++) a1[0][j] = (short)(row < g.M ? f2bf(g.X[(size_t)row * kPIn + q + j]) : 0);
+            for (int j = 0; j < 4; j++) a1[0][j] = (short)(row < g.M ? f2bf(g.X[(size_t)row * kIn + q + j]) : 0);
         }
-        predict_layer<1, kPH / 16, false>(a1, sw + kPW1, sb, tile, nullptr, row0, g.M);
-        bf16x4 a[kPH / 16];
+        predict_layer<1, kHid / 16, false>(a1, sw + kPW1, sb, tile, nullptr, row0, g.M);
+        bf16x4 a[kHid / 16];
         // (LDS operations of one wave complete in order; the fence keeps the compiler's order)
         __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
 #pragma unroll
-        for (int kc = 0; kc < kPH / 16; kc++) a[kc] = *(const bf16x4*)(tile + r * kPTileRow + kc * 16 + q);
+        for (int kc = 0; kc < kHid / 16; kc++) a[kc] = *(const bf16x4*)(tile + r * kPTileRow + kc * 16 + q);
         __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-        predict_layer<kPH / 16, kPH / 16, false>(a, sw + kPW2, sb + kPH, tile, nullptr, row0, g.M);
-        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-#pragma unroll
-        for (int kc = 0; kc < kPH / 16; kc++) a[kc] = *(const bf16x4*)(tile + r * kPTileRow + kc * 16 + q);
-        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-        predict_layer<kPH / 16, kPH / 16, false>(a, sw + kPW3, sb + 2 * kPH, tile, nullptr, row0, g.M);
+        predict_layer<kHid / 16, kHid / 16, false>(a, sw + kPW2, sb + kHid, tile, nullptr, row0, g.M);
         __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
 #pragma unroll
-        for (int kc = 0; kc < kPH / 16; kc++) a[kc] = *(const bf16x4*)(tile + r * kPTileRow + kc * 16 + q);
+        for (int kc = 0; kc < kHid / 16; kc++) a[kc] = *(const bf16x4*)(tile + r * kPTileRow + kc * 16 + q);
         __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-        predict_layer<kPH / 16, kPOut / 16, true>(a, sw + kPW4, sb + 3 * kPH, tile, g.Y, row0, g.M);
+        predict_layer<kHid / 16, kHid / 16, false>(a, sw + kPW3, sb + 2 * kHid, tile, nullptr, row0, g.M);
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+#pragma unroll
+        for (int kc = 0; kc < kHid / 16; kc++) a[kc] = *(const bf16x4*)(tile + r * kPTileRow + kc * 16 + q);
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        predict_layer<kHid / 16, kOut / 16, true>(a, sw + kPW4, sb + 3 * kHid, tile, g.Y, row0, g.M);
     }
+}
+
+// ---- training: loss and gradients of a batch in one kernel ------------------------------------
+// A workgroup of 8 waves takes 32 rows at a time through the forward pass, the loss and the backward
+// pass without leaving the CU: four waves share a 16-row tile and own a quarter of every layer's
+// outputs, and the tanh outputs (FP32) stay in their registers until the backward pass needs them.
+// Operands change layout through LDS, where each layer's inputs and gradients lie twice: row-major
+// (the operand of the products that reduce over inputs or outputs) and transposed with 4 consecutive
+// rows per lane (the operand of the weight gradients, which reduce over the rows; the MFMA result
+// layout writes it directly).  The weight gradients are 152 tiles of 16 x 16, 19 per wave,
+// accumulated in registers over all rows of the workgroup and written once, to the workgroup's own
+// slice of a partial-sum buffer that reduce_grad_kernel adds up (no atomics: the sums do not depend
+// on the order in which workgroups finish).
+// What bounds it: 8192 rows need 2 GFLOP of matrix work, under 2 us of the matrix cores; a workgroup's
+// time is its serial chain of 8 layer products (tanh, LDS round trips and barriers, weight fragments
+// from L2) and the write of its 157 KB slice.  32 rows per workgroup put 8192 rows on all 256 CUs:
+// 39 us for the kernel and 9 us for the sums, against 59 and 6 us with 64 rows (half the CUs) and
+// 780 us in 21 launches with one GEMM launch per product, whose weight gradients (one wave per tile,
+// 1024 rows each) took 590 us.
+constexpr int kTWaves = 8, kTRows = 32;
+constexpr int kTSplit = kTWaves / (kTRows / 16);  // waves that share a 16-row tile
+constexpr int kTNt = kHid / 16 / kTSplit;         // tiles of 16 outputs a wave owns in a hidden layer
+constexpr int kTRow = kHid + kPad;   // elements per row of the row-major tile
+constexpr int kTCol = kTRows + kPad; // elements per column of the transposed tiles
+constexpr int kTBias = 3 * kHid + kOut;
+constexpr int kPartStride = kNumParams + 4;  // a workgroup's gradients, then its loss
+constexpr int kTMaxBlocks = 256;
+
+struct TrainArgs {
+    const uint16_t* p16;   // BF16 parameters, weights as [in][out]
+    const uint16_t* p16t;  // weights as [out][in]
+    const float* p;
+    const float* X;        // [M][16]
+    const float* T;        // [M][32]
+    const float* w;        // [32]
+    float* part;           // [gridDim.x][kPartStride]
+    int M;
+};
+
+// Operand fragments of NT tiles of 16 output columns, from W stored with the reduction contiguous.
+template <int KC, int NT>
+__device__ __forceinline__ void load_frags(const uint16_t* W, int col0, bf16x4 (&b)[NT][KC]) {
+    const int lane = threadIdx.x & 63, r = lane & 15, q = (lane >> 4) << 2;
+#pragma unroll
+    for (int nt = 0; nt < NT; nt++)
+#pragma unroll
+        for (int kc = 0; kc < KC; kc++)
+            b[nt][kc] = *(const bf16x4*)(W + (size_t)(col0 + nt * 16 + r) * (KC * 16) + kc * 16 + q);
+}
+// acc = A B over KC slices of 16, A from the row-major tile (rows row0..row0+15).
+template <int KC, int NT>
+__device__ __forceinline__ void tile_product(const uint16_t* tile, int row0, const bf16x4 (&b)[NT][KC], f32x4 (&acc)[NT]) {
+    const int lane = threadIdx.x & 63, r = lane & 15, q = (lane >> 4) << 2;
+    bf16x4 a[KC];
+#pragma unroll
+    for (int kc = 0; kc < KC; kc++) a[kc] = *(const bf16x4*)(tile + (row0 + r) * kTRow + kc * 16 + q);
+#pragma unroll
+    for (int nt = 0; nt < NT; nt++) acc[nt] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int kc = 0; kc < KC; kc++)
+#pragma unroll
+        for (int nt = 0; nt < NT; nt++) acc[nt] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(a[kc], b[nt][kc], acc[nt], 0, 0, 0);
+}
+// acc[i] += In^T D for the 16 inputs at in0 and the 16-column tiles out0 + 16 i, over the rows.
+template <int NT>
+__device__ __forceinline__ void weight_grad(const uint16_t* inT, int in0, const uint16_t* dT, int out0, f32x4 (&acc)[NT]) {
+    const int lane = threadIdx.x & 63, r = lane & 15, q = (lane >> 4) << 2;
+#pragma unroll
+    for (int kc = 0; kc < kTRows / 16; kc++) {
+        const bf16x4 a = *(const bf16x4*)(inT + (in0 + r) * kTCol + kc * 16 + q);
+#pragma unroll
+        for (int nt = 0; nt < NT; nt++) {
+            const bf16x4 b = *(const bf16x4*)(dT + (out0 + nt * 16 + r) * kTCol + kc * 16 + q);
+            acc[nt] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(a, b, acc[nt], 0, 0, 0);
+        }
+    }
+}
+// A wave's columns col0.. of its 16-row tile: to the row-major tile and / or transposed.
+template <int NT>
+__device__ __forceinline__ void put_rows(uint16_t* tile, int row0, int col0, const f32x4 (&v)[NT]) {
+    const int lane = threadIdx.x & 63, r = lane & 15, q = (lane >> 4) << 2;
+#pragma unroll
+    for (int nt = 0; nt < NT; nt++)
+#pragma unroll
+        for (int j = 0; j < 4; j++) tile[(row0 + q + j) * kTRow + col0 + nt * 16 + r] = f2bf(v[nt][j]);
+}
+template <int NT>
+__device__ __forceinline__ void put_cols(uint16_t* tileT, int row0, int col0, const f32x4 (&v)[NT]) {
+    const int lane = threadIdx.x & 63, r = lane & 15, q = (lane >> 4) << 2;
+#pragma unroll
+    for (int nt = 0; nt < NT; nt++) {
+        bf16x4 h;
+#pragma unroll
+        for (int j = 0; j < 4; j++) h[j] = (short)f2bf(v[nt][j]);
+        *(bf16x4*)(tileT + (col0 + nt * 16 + r) * kTCol + row0 + q) = h;
+    }
+}
+// Gradient through tanh from its output H, and this lane's share of the bias gradients.
+__device__ __forceinline__ void tanh_grad(f32x4 (&d)[kTNt], const f32x4 (&H)[kTNt], float (&db)[kTNt]) {
+#pragma unroll
+    for (int nt = 0; nt < kTNt; nt++)
+#pragma unroll
+        for (int j = 0; j < 4; j++) {
+            d[nt][j] *= 1.f - H[nt][j] * H[nt][j];
+            db[nt] += d[nt][j];
+        }
+}
+__device__ __forceinline__ void tanh_layer(f32x4 (&H)[kTNt], const float* bias, int col0) {
+    const int r = threadIdx.x & 15;
+#pragma unroll
+    for (int nt = 0; nt < kTNt; nt++) {
+        const float bc = bias[col0 + nt * 16 + r];
+#pragma unroll
+        for (int j = 0; j < 4; j++) H[nt][j] = tanhf(H[nt][j] + bc);
+    }
+}
+
+__global__ void __launch_bounds__(64 * kTWaves) mlp_train_kernel(TrainArgs args) {
+    __shared__ __align__(16) uint16_t s_tile[kTRows * kTRow];
+    __shared__ __align__(16) uint16_t s_inT[kHid * kTCol], s_dT[kHid * kTCol], s_xT[kIn * kTCol];
+    __shared__ float s_loss[kTWaves];
+    const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+    const int r = lane & 15, q = (lane >> 4) << 2;
+    const int row0 = wave / kTSplit * 16, share = wave % kTSplit, col0 = share * kTNt * 16;
+    const bool outs = share < kOut / 16;  // this wave owns a tile of the output layer
+    f32x4 gw1[1] = {}, gw2[8] = {}, gw3[8] = {}, gw4[2] = {};
+    float db1[kTNt] = {}, db2[kTNt] = {}, db3[kTNt] = {}, db4 = 0.f, loss = 0.f;
+    TrainArgs g = args;
+    for (int base = blockIdx.x * kTRows; base < args.M; base += gridDim.x * kTRows) {
+        // (opaque per trip: the weight fragments are the same for every 64 rows, and hoisted out of
+        // the loop they would not fit the registers)
+        int zero = 0;
+        asm volatile("" : "+s"(zero));
+        g.p16 = args.p16 + zero;
+        g.p16t = args.p16t + zero;
+        g.p = args.p + zero;
+        f32x4 H1[kTNt], H2[kTNt], H3[kTNt];
+        {
+            const int row = base + row0 + r;
+            bf16x4 a;
+#pragma unroll
+            for (int j = 0; j < 4; j++) a[j] = (short)(row < g.M ? f2bf(g.X[(size_t)row * kIn + q + j]) : 0);
+            bf16x4 b[kTNt][1];
+            load_frags<1, kTNt>(g.p16t + kOff1, col0, b);
+            if (share == 0) {
+#pragma unroll
+                for (int j = 0; j < 4; j++) s_xT[(q + j) * kTCol + row0 + r] = (uint16_t)a[j];
+            }
+#pragma unroll
+            for (int nt = 0; nt < kTNt; nt++)
+                H1[nt] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(a, b[nt][0], (f32x4{0.f, 0.f, 0.f, 0.f}), 0, 0, 0);
+        }
+        tanh_layer(H1, g.p + kOff1 + kIn * kHid, col0);
+        put_rows(s_tile, row0, col0, H1);
+        {
+            bf16x4 b[kTNt][8];
+            load_frags<8, kTNt>(g.p16t + kOff2, col0, b);
+            __syncthreads();
+            tile_product<8, kTNt>(s_tile, row0, b, H2);
+        }
+        tanh_layer(H2, g.p + kOff2 + kHid * kHid, col0);
+        __syncthreads();
+        put_rows(s_tile, row0, col0, H2);
+        {
+            bf16x4 b[kTNt][8];
+            load_frags<8, kTNt>(g.p16t + kOff3, col0, b);
+            __syncthreads();
+            tile_product<8, kTNt>(s_tile, row0, b, H3);
+        }
+        tanh_layer(H3, g.p + kOff3 + kHid * kHid, col0);
+        __syncthreads();
+        put_rows(s_tile, row0, col0, H3);
+        put_cols(s_inT, row0, col0, H3);
+        // output layer and loss: dY = 2 w (Y - T) / M (0 past the batch)
+        f32x4 dY[1] = {};
+        __syncthreads();
+        if (outs) {
+            bf16x4 b[1][8];
+            load_frags<8, 1>(g.p16t + kOff4, share * 16, b);
+            tile_product<8, 1>(s_tile, row0, b, dY);
+            const int col = share * 16 + r;
+            const float bc = g.p[kOff4 + kHid * kOut + col], wc = g.w[col];
+#pragma unroll
+            for (int j = 0; j < 4; j++) {
+                const int row = base + row0 + q + j;
+                float d = 0.f;
+                if (row < g.M) d = (dY[0][j] + bc) - g.T[(size_t)row * kOut + col];
+                loss += wc * d * d;
+                dY[0][j] = 2.f * wc * d / (float)g.M;
+                db4 += dY[0][j];
+            }
+        }
+        __syncthreads();
+        // backward: the layers' gradients with respect to their pre-activations replace the tile
+        f32x4 D[kTNt];
+        if (outs) {
+            put_rows(s_tile, row0, share * 16, dY);
+            put_cols(s_dT, row0, share * 16, dY);
+        }
+        {
+            bf16x4 b[kTNt][2];
+            load_frags<2, kTNt>(g.p16 + kOff4, col0, b);
+            __syncthreads();
+            tile_product<2, kTNt>(s_tile, row0, b, D);
+        }
+        weight_grad<2>(s_inT, wave * 16, s_dT, 0, gw4);
+        tanh_grad(D, H3, db3);
+        __syncthreads();
+        put_rows(s_tile, row0, col0, D);
+        put_cols(s_dT, row0, col0, D);
+        put_cols(s_inT, row0, col0, H2);
+        {
+            bf16x4 b[kTNt][8];
+            load_frags<8, kTNt>(g.p16 + kOff3, col0, b);
+            __syncthreads();
+            tile_product<8, kTNt>(s_tile, row0, b, D);
+        }
+        weight_grad<8>(s_inT, wave * 16, s_dT, 0, gw3);
+        tanh_grad(D, H2, db2);
+        __syncthreads();
+        put_rows(s_tile, row0, col0, D);
+        put_cols(s_dT, row0, col0, D);
+        put_cols(s_inT, row0, col0, H1);
+        {
+            bf16x4 b[kTNt][8];
+            load_frags<8, kTNt>(g.p16 + kOff2, col0, b);
+            __syncthreads();
+            tile_product<8, kTNt>(s_tile, row0, b, D);
+        }
+        weight_grad<8>(s_inT, wave * 16, s_dT, 0, gw2);
+        tanh_grad(D, H1, db1);
+        __syncthreads();
+        put_cols(s_dT, row0, col0, D);
+        __syncthreads();
+        weight_grad<1>(s_xT, 0, s_dT, wave * 16, gw1);
+        __syncthreads();
+    }
+    // this workgroup's sums
+    float* const out = args.part + (size_t)blockIdx.x * kPartStride;
+#pragma unroll
+    for (int j = 0; j < 4; j++) {
+        out[kOff1 + (q + j) * kHid + wave * 16 + r] = gw1[0][j];
+        const int in = wave * 16 + q + j;
+#pragma unroll
+        for (int nt = 0; nt < 8; nt++) {
+            out[kOff2 + in * kHid + nt * 16 + r] = gw2[nt][j];
+            out[kOff3 + in * kHid + nt * 16 + r] = gw3[nt][j];
+        }
+#pragma unroll
+        for (int nt = 0; nt < 2; nt++) out[kOff4 + in * kOut + nt * 16 + r] = gw4[nt][j];
+    }
+    // bias gradients: over a tile's rows by lane exchange, over the four tiles through LDS
+    float* const s_db = (float*)s_inT;  // [kTRows / 16][kTBias]
+    auto put_bias = [&](float v, int at) {
+        v += __shfl_xor(v, 16, 64);
+        v += __shfl_xor(v, 32, 64);
+        if (lane < 16) s_db[wave / kTSplit * kTBias + at + r] = v;
+    };
+#pragma unroll
+    for (int nt = 0; nt < kTNt; nt++) {
+        put_bias(db1[nt], col0 + nt * 16);
+        put_bias(db2[nt], kHid + col0 + nt * 16);
+        put_bias(db3[nt], 2 * kHid + col0 + nt * 16);
+    }
+    if (outs) put_bias(db4, 3 * kHid + share * 16);
+    for (int m = 32; m >= 1; m >>= 1) loss += __shfl_xor(loss, m, 64);
+    if (lane == 0) s_loss[wave] = loss;
+    __syncthreads();
+    for (int i = threadIdx.x; i < kTBias; i += blockDim.x) {
+        const int l = i >> 7, c = i & 127;
+        const int at = l == 0 ? kOff2 - kHid : (l == 1 ? kOff3 - kHid : (l == 2 ? kOff4 - kHid : kNumParams - kOut));
+        float v = s_db[i];
+        for (int k = 1; k < kTRows / 16; k++) v += s_db[k * kTBias + i];
+        out[at + c] = v;
+    }
+    if (threadIdx.x == 0) {
+        float t = 0.f;
+        for (int k = 0; k < kTWaves; k++) t += s_loss[k];
+        out[kNumParams] = t;
+    }
+}
+
+// Gradients and loss from the workgroups' sums: 64 groups of four parameters per block, each
+// summed by four waves that take every fourth workgroup's slice (the slices stream from L2; one
+// thread per group alone would leave the loads of 128 slices in a chain).
+__global__ void __launch_bounds__(256) reduce_grad_kernel(const float* __restrict__ part, int nblocks, int M, float* grad,
+                                                          float* loss) {
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int e = (blockIdx.x * 64 + lane) * 4;
+    f32x4 s = {0.f, 0.f, 0.f, 0.f};
+    if (e < kPartStride) {
+#pragma unroll 8
+        for (int b = wave; b < nblocks; b += 4) s += *(const f32x4*)(part + (size_t)b * kPartStride + e);
+    }
+    __shared__ f32x4 acc[4][64];
+    acc[wave][lane] = s;
+    __syncthreads();
+    if (wave != 0) return;
+    s = (acc[0][lane] + acc[1][lane]) + (acc[2][lane] + acc[3][lane]);
+    if (e < kNumParams) *(f32x4*)(grad + e) = s;
+    else if (e == kNumParams) *loss = s[0] / (float)M;
 }
 
 }  // namespace assist_gpu
@@ -323,14 +505,6 @@ bool ok(hipError_t e, const char* what) {
     return false;
 }
 
-template <typename TAe, typename TBe, bool TA, bool TB>
-hipError_t gemm(const GemmArgs& g, int zsplit, hipStream_t s) {
-    const int tiles = ((g.M + 15) / 16) * ((g.N + 15) / 16);
-    dim3 grid((tiles + 3) / 4, 1, zsplit);
-    hipLaunchKernelGGL((gemm_bf16_kernel<TAe, TBe, TA, TB>), grid, dim3(256), 0, s, g);
-    return hipGetLastError();
-}
-
 unsigned grid1(size_t n) { return (unsigned)((n + 255) / 256); }
 
 }  // namespace
@@ -339,25 +513,29 @@ struct assist_mlp {
     int device = 0;
     int max_batch = 0;
     float* p = nullptr;      // FP32 master parameters
-    uint16_t* p16 = nullptr; // BF16 weights for the matrix cores
+    uint16_t* p16 = nullptr; // BF16 weights for the matrix cores, [in][out]
+    uint16_t* p16t = nullptr; // and [out][in]
     float* g = nullptr;      // gradients
     float* m = nullptr;      // Adam moments
     float* v = nullptr;
-    float* act = nullptr;    // H1, H2, H3, Y: max_batch x (3 * hidden + out)
-    float* dact = nullptr;   // dH (max_batch x hidden) x 2 ping-pong + dY
+    float* part = nullptr;   // gradients and loss per workgroup of the training kernel
     float* wout = nullptr;   // output weights of the loss [out]
     float* loss = nullptr;   // [1]
 };
 
 static void mlp_release(assist_mlp* n) {
     if (!n) return;
-    for (void* q : {(void*)n->p, (void*)n->p16, (void*)n->g, (void*)n->m, (void*)n->v, (void*)n->act, (void*)n->dact,
+    for (void* q : {(void*)n->p, (void*)n->p16, (void*)n->p16t, (void*)n->g, (void*)n->m, (void*)n->v, (void*)n->part,
                     (void*)n->wout, (void*)n->loss})
         if (q) (void)hipFree(q);
     delete n;
 }
 
-static size_t act_stride(int max_batch) { return (size_t)max_batch; }
+// Workgroups of the training kernel for M rows.
+static int train_blocks(int M) {
+    const int b = (M + kTRows - 1) / kTRows;
+    return b < kTMaxBlocks ? b : kTMaxBlocks;
+}
 
 extern "C" {
 
@@ -368,13 +546,13 @@ struct assist_mlp* assist_mlp_create(int max_batch, unsigned long long seed) {
     auto* n = new assist_mlp();
     n->max_batch = max_batch;
     const size_t np = w_off(kLayers);
-    const size_t H = ASSIST_MLP_HIDDEN, O = ASSIST_MLP_OUT;
-    const size_t B = act_stride(max_batch);
+    const size_t O = ASSIST_MLP_OUT;
     bool good = ok(hipGetDevice(&n->device), "hipGetDevice") && ok(hipMalloc(&n->p, np * 4), "hipMalloc") &&
-                ok(hipMalloc(&n->p16, np * 2), "hipMalloc") && ok(hipMalloc(&n->g, np * 4), "hipMalloc") &&
+                ok(hipMalloc(&n->p16, np * 2), "hipMalloc") && ok(hipMalloc(&n->p16t, np * 2), "hipMalloc") &&
+                ok(hipMalloc(&n->g, np * 4), "hipMalloc") &&
                 ok(hipMalloc(&n->m, np * 4), "hipMalloc") && ok(hipMalloc(&n->v, np * 4), "hipMalloc") &&
-                ok(hipMalloc(&n->act, B * (3 * H + O) * 4), "hipMalloc") &&
-                ok(hipMalloc(&n->dact, B * (2 * H + O) * 4), "hipMalloc") && ok(hipMalloc(&n->wout, O * 4), "hipMalloc") &&
+                ok(hipMalloc(&n->part, (size_t)train_blocks(max_batch) * kPartStride * 4), "hipMalloc") &&
+                ok(hipMalloc(&n->wout, O * 4), "hipMalloc") &&
                 ok(hipMalloc(&n->loss, 4), "hipMalloc");
     if (!good) {
         mlp_release(n);
@@ -409,7 +587,7 @@ int assist_mlp_set_params(struct assist_mlp* n, const float* host) {
     if (!ok(hipMemcpy(n->p, host, np * 4, hipMemcpyHostToDevice), "hipMemcpy") ||
         !ok(hipMemset(n->m, 0, np * 4), "hipMemset") || !ok(hipMemset(n->v, 0, np * 4), "hipMemset"))
         return ASSIST_BATCH_ERROR_DEVICE;
-    hipLaunchKernelGGL(to_bf16_kernel, dim3(grid1(np)), dim3(256), 0, 0, n->p, n->p16, np);
+    hipLaunchKernelGGL(to_bf16_kernel, dim3(grid1(np)), dim3(256), 0, 0, n->p, n->p16, n->p16t, (int)np);
     if (!ok(hipGetLastError(), "to_bf16") || !ok(hipDeviceSynchronize(), "to_bf16")) return ASSIST_BATCH_ERROR_DEVICE;
     return 0;
 }
@@ -425,41 +603,7 @@ int assist_mlp_set_output_weights(struct assist_mlp* n, const float* host_w) {
                                                                                               : ASSIST_BATCH_ERROR_DEVICE;
 }
 
-// Forward pass of M rows (M <= max_batch): d_X [M][16] -> d_Y [M][32] (device pointers).  The
-// hidden activations stay in the network's workspace for a following backward pass.
-int assist_mlp_forward(struct assist_mlp* n, const float* d_X, int M, float* d_Y, void* stream) {
-    if (!n || !d_X || M < 0 || M > n->max_batch) return ASSIST_BATCH_ERROR_ARG;
-    if (M == 0) return 0;
-    hipStream_t s = (hipStream_t)stream;
-    const int H = ASSIST_MLP_HIDDEN;
-    const size_t B = act_stride(n->max_batch);
-    const float* in = d_X;
-    int ld_in = ASSIST_MLP_IN;
-    for (int l = 0; l < kLayers; l++) {
-        GemmArgs g;
-        memset(&g, 0, sizeof g);
-        g.M = M;
-        g.N = kDims[l + 1];
-        g.K = kDims[l];
-        g.A = in;
-        g.lda = ld_in;
-        g.B = n->p16 + w_off(l);
-        g.ldb = kDims[l + 1];
-        float* out = (l < kLayers - 1) ? n->act + (size_t)l * B * H : (d_Y ? d_Y : n->act + 3 * B * H);
-        g.C = out;
-        g.ldc = kDims[l + 1];
-        g.bias = n->p + b_off(l);
-        g.act = (l < kLayers - 1) ? kActTanh : kActNone;
-        g.kchunk = ((g.K + 15) / 16) * 16;
-        if (!ok(gemm<float, uint16_t, false, false>(g, 1, s), "mlp forward")) return ASSIST_BATCH_ERROR_DEVICE;
-        in = out;
-        ld_in = kDims[l + 1];
-    }
-    return 0;
-}
-
-// Prediction forward pass of any number of rows: d_X [M][16] -> d_Y [M][32], keeping no
-// activations (the fused kernel above; outputs equal assist_mlp_forward's bit for bit).
+// Forward pass of any number of rows: d_X [M][16] -> d_Y [M][32].
 int assist_mlp_predict(struct assist_mlp* n, const float* d_X, int M, float* d_Y, void* stream) {
     if (!n || !d_X || !d_Y || M < 0) return ASSIST_BATCH_ERROR_ARG;
     if (M == 0) return 0;
@@ -472,7 +616,7 @@ int assist_mlp_predict(struct assist_mlp* n, const float* d_X, int M, float* d_Y
         !ok(hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, dev), "hipDeviceGetAttribute"))
         return ASSIST_BATCH_ERROR_DEVICE;
     PredictArgs g;
-    g.p16 = n->p16;
+    g.p16t = n->p16t;
     g.p = n->p;
     g.X = d_X;
     g.Y = d_Y;
@@ -486,77 +630,35 @@ int assist_mlp_predict(struct assist_mlp* n, const float* d_X, int M, float* d_Y
     return ok(hipGetLastError(), "mlp predict") ? 0 : ASSIST_BATCH_ERROR_DEVICE;
 }
 
+// Forward pass of at most max_batch rows (the same kernel; nothing to do without an output).
+int assist_mlp_forward(struct assist_mlp* n, const float* d_X, int M, float* d_Y, void* stream) {
+    if (!n || !d_X || M < 0 || M > n->max_batch) return ASSIST_BATCH_ERROR_ARG;
+    return d_Y ? assist_mlp_predict(n, d_X, M, d_Y, stream) : 0;
+}
+
 // Forward and backward pass of the weighted squared error against d_T [M][32]; leaves the
 // gradients in the network (and copies them to host_grad when given) and returns the loss.
 int assist_mlp_loss_grad(struct assist_mlp* n, const float* d_X, const float* d_T, int M, float* loss,
                          float* host_grad, void* stream) {
     if (!n || !d_X || !d_T || M <= 0 || M > n->max_batch) return ASSIST_BATCH_ERROR_ARG;
     hipStream_t s = (hipStream_t)stream;
-    const int H = ASSIST_MLP_HIDDEN, O = ASSIST_MLP_OUT;
-    const size_t B = act_stride(n->max_batch);
-    const size_t np = w_off(kLayers);
-    float* Y = n->act + 3 * B * H;
-    int rc = assist_mlp_forward(n, d_X, M, nullptr, stream);
-    if (rc) return rc;
-    hipLaunchKernelGGL(fill_kernel, dim3(grid1(np)), dim3(256), 0, s, n->g, np, 0.f);
-    hipLaunchKernelGGL(fill_kernel, dim3(1), dim3(256), 0, s, n->loss, (size_t)1, 0.f);
-    float* dY = n->dact + 2 * B * H;
-    hipLaunchKernelGGL(mse_kernel, dim3(256), dim3(256), 0, s, (const float*)Y, d_T, (const float*)n->wout, M, O, dY,
-                       n->loss);
-    if (!ok(hipGetLastError(), "mse")) return ASSIST_BATCH_ERROR_DEVICE;
-    // walk the layers backwards; dcur = gradient w.r.t. the pre-activation of layer l's output
-    float* dcur = dY;
-    for (int l = kLayers - 1; l >= 0; l--) {
-        const int K = kDims[l], N = kDims[l + 1];
-        const float* Hin = (l == 0) ? d_X : n->act + (size_t)(l - 1) * B * H;
-        const int ld_in = K;
-        // dW_l = Hin^T dcur  (reduction over the batch, split over blockIdx.z)
-        {
-            GemmArgs g;
-            memset(&g, 0, sizeof g);
-            g.M = K;
-            g.N = N;
-            g.K = M;
-            g.A = Hin;
-            g.lda = ld_in;
-            g.B = dcur;
-            g.ldb = N;
-            g.C = n->g + w_off(l);
-            g.ldc = N;
-            g.atomic = 1;
-            const int zs = (M + 1023) / 1024;
-            g.kchunk = ((M + zs - 1) / zs + 15) / 16 * 16;
-            const int zsplit = (M + g.kchunk - 1) / g.kchunk;
-            if (!ok(gemm<float, float, true, false>(g, zsplit, s), "mlp dW")) return ASSIST_BATCH_ERROR_DEVICE;
-        }
-        // db_l = column sums of dcur
-        hipLaunchKernelGGL(colsum_kernel, dim3((M + 1023) / 1024, N), dim3(256), 0, s, (const float*)dcur, M, N,
-                           n->g + b_off(l));
-        if (!ok(hipGetLastError(), "colsum")) return ASSIST_BATCH_ERROR_DEVICE;
-        if (l == 0) break;
-        // dHin = dcur W_l^T, then through tanh
-        float* dnext = n->dact + (size_t)(l % 2) * B * H;
-        GemmArgs g;
-        memset(&g, 0, sizeof g);
-        g.M = M;
-        g.N = K;
-        g.K = N;
-        g.A = dcur;
-        g.lda = N;
-        g.B = n->p16 + w_off(l);
-        g.ldb = N;  // W stored [K][N]; element (k = n_idx, j = k_idx) of W^T is W[j * N + k]
-        g.C = dnext;
-        g.ldc = K;
-        g.kchunk = ((N + 15) / 16) * 16;
-        if (!ok(gemm<float, uint16_t, false, true>(g, 1, s), "mlp dX")) return ASSIST_BATCH_ERROR_DEVICE;
-        const size_t cnt = (size_t)M * K;
-        hipLaunchKernelGGL(tanh_backward_kernel, dim3(grid1(cnt)), dim3(256), 0, s, dnext,
-                           (const float*)(n->act + (size_t)(l - 1) * B * H), cnt);
-        if (!ok(hipGetLastError(), "tanh backward")) return ASSIST_BATCH_ERROR_DEVICE;
-        dcur = dnext;
-    }
+    TrainArgs g;
+    g.p16 = n->p16;
+    g.p16t = n->p16t;
+    g.p = n->p;
+    g.X = d_X;
+    g.T = d_T;
+    g.w = n->wout;
+    g.part = n->part;
+    g.M = M;
+    const int blocks = train_blocks(M);
+    hipLaunchKernelGGL(mlp_train_kernel, dim3(blocks), dim3(64 * kTWaves), 0, s, g);
+    if (!ok(hipGetLastError(), "mlp train")) return ASSIST_BATCH_ERROR_DEVICE;
+    hipLaunchKernelGGL(reduce_grad_kernel, dim3((kPartStride / 4 + 63) / 64), dim3(256), 0, s, (const float*)n->part,
+                       blocks, M, n->g, n->loss);
+    if (!ok(hipGetLastError(), "mlp reduce")) return ASSIST_BATCH_ERROR_DEVICE;
     if (loss && !ok(hipMemcpyAsync(loss, n->loss, 4, hipMemcpyDeviceToHost, s), "hipMemcpyAsync")) return ASSIST_BATCH_ERROR_DEVICE;
-    if (host_grad && !ok(hipMemcpyAsync(host_grad, n->g, np * 4, hipMemcpyDeviceToHost, s), "hipMemcpyAsync"))
+    if (host_grad && !ok(hipMemcpyAsync(host_grad, n->g, (size_t)kNumParams * 4, hipMemcpyDeviceToHost, s), "hipMemcpyAsync"))
         return ASSIST_BATCH_ERROR_DEVICE;
     if (!ok(hipStreamSynchronize(s), "mlp backward")) return ASSIST_BATCH_ERROR_DEVICE;
     return 0;
@@ -566,8 +668,8 @@ int assist_mlp_adam_step(struct assist_mlp* n, float lr, float beta1, float beta
     if (!n || step < 1) return ASSIST_BATCH_ERROR_ARG;
     const size_t np = w_off(kLayers);
     const float c1 = 1.f - powf(beta1, (float)step), c2 = 1.f - powf(beta2, (float)step);
-    hipLaunchKernelGGL(adam_kernel, dim3(grid1(np)), dim3(256), 0, (hipStream_t)stream, n->p, n->p16, (const float*)n->g,
-                       n->m, n->v, np, lr, beta1, beta2, eps, c1, c2);
+    hipLaunchKernelGGL(adam_kernel, dim3(grid1(np)), dim3(256), 0, (hipStream_t)stream, n->p, n->p16, n->p16t,
+                       (const float*)n->g, n->m, n->v, (int)np, lr, beta1, beta2, eps, c1, c2);
     return ok(hipGetLastError(), "adam") ? 0 : ASSIST_BATCH_ERROR_DEVICE;
 }
 

@@ -471,7 +471,7 @@ int assist_device_synchronize(void);
 
 struct assist_mlp;
 int assist_mlp_num_params(void);
-/* Workspace for batches of up to max_batch rows; Glorot-uniform weights from `seed`. */
+/* Workspace for training batches of up to max_batch rows; Glorot-uniform weights from `seed`. */
 struct assist_mlp* assist_mlp_create(int max_batch, unsigned long long seed);
 void assist_mlp_free(struct assist_mlp* net);
 int assist_mlp_max_batch(const struct assist_mlp* net);
@@ -482,8 +482,7 @@ int assist_mlp_get_params(const struct assist_mlp* net, float* host);
 int assist_mlp_set_output_weights(struct assist_mlp* net, const float* host_w);
 /* d_X[M][16] -> d_Y[M][32] (device pointers, M <= max_batch). */
 int assist_mlp_forward(struct assist_mlp* net, const float* d_X, int M, float* d_Y, void* stream);
-/* The same outputs, bit for bit, for any M, keeping no activations (one fused kernel: the
- * prediction path of assist_batch_predict_start). */
+/* The same for any M (one fused kernel: the prediction path of assist_batch_predict_start). */
 int assist_mlp_predict(struct assist_mlp* net, const float* d_X, int M, float* d_Y, void* stream);
 /* Forward and backward pass of the loss against d_T[M][32]; gradients stay on the device
  * (host_grad, if given, receives a copy) and *loss receives the loss. */
