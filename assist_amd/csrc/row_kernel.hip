@@ -25,7 +25,7 @@
 // wave.  Two waves per SIMD overlap theirs, and the ephemeris tables leave LDS for six waves per CU.
 // Measured on an MI355X against the 8-lane kernel: one system, FP64, 1.95 us per evaluation (4.67)
 // alone and 3.3 us (5.5) with 6 vectors; 4,096 x 7 vectors over 3,650 d 37 ms (61); 262,144 x 7 over
-// 365 d in the mixed form 119 ms (143); 65,536 uneven real-only spans up to 10,000 d 157 ms (297).
+// 365 d in the mixed form 104 ms (143); 65,536 uneven real-only spans up to 10,000 d 152 ms (297).
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
@@ -375,6 +375,16 @@ __device__ __forceinline__ void row_force_eval(const DevEphem& E, const ForceOpt
 }
 
 enum : int { kRowNone = 0, kRowSetup = 1, kRowFinish = 2 };
+// Mixed form: a row about to evaluate the last substep of a pass waits for rows of its wave that are at
+// most this many substeps behind.  Most attempts take one pass there (8 evaluations with the step's
+// start), and a step's end, the prediction of the next and its ephemeris cost about as many
+// instructions as 3 evaluations, which the wave issues once for all the rows that get there together:
+// waiting aligns the rows for good, since a second pass (7 evaluations) leaves a row one behind.
+// Measured without and with waits of at most 1 and 2: 65,536 x 7 vectors over 100 d 17.3, 14.5,
+// 14.6 ms, real particles alone 10.8, 9.4, 9.4 ms (3 to 6 give no more).  The FP64 form's attempts
+// take two to four passes and drift apart again: 65,536 real particles over 60 d 9.9, 9.8, 9.7 ms,
+// 4,096 x 7 over 300 d 4.85, 5.1, 5.2 ms.
+constexpr int kRowAlign = 2;
 
 // NV: vectors per lane quad (1: up to 4 vectors per system, 2: up to 8).  Jacobian: the systems
 // carry variational vectors.
@@ -629,7 +639,13 @@ ias15_row_kernel(IntegrateArgs args) {
             __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
             need_eph = false;
         }
-        if (!active || todo == kRowFinish) continue;
+        bool wait = false;
+        if constexpr (Mixed) {
+            // (a row that is waited for never waits itself, so each trip brings one nearer)
+            const bool behind = active && todo != kRowFinish && phase && n < 7 && n >= 7 - kRowAlign;
+            wait = __ballot(behind) != 0ULL && phase && n == 7;
+        }
+        if (!active || todo == kRowFinish || wait) continue;
         // ---- evaluation point of this trip ----
         double xe[NV], ve[NV], te;
         if (!phase) {
