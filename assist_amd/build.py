@@ -23,7 +23,7 @@ ROCM = os.environ.get("ROCM_PATH", "/opt/rocm")
 HIPCC = os.path.join(ROCM, "bin", "hipcc")
 ARCH = os.environ.get("ASSIST_AMD_ARCH", "gfx950")
 
-HIP_SOURCES = ["kernels.hip", "row_kernel.hip", "mlp.hip"]
+HIP_SOURCES = ["kernels.hip", "row_kernel.hip", "lane_kernel.hip", "mlp.hip"]
 CPP_SOURCES = ["spk.cpp", "ascii.cpp", "assist_api.cpp", "batch.cpp"]
 HEADERS = ["device_types.h", "force_model.h", "force_terms64.h", "ias15_device.h", "ias15_tables.h", "kernels.h", "internal.h"]
 
@@ -33,7 +33,8 @@ HIP_FLAGS = ["--offload-arch=" + ARCH, "-O3", "-std=c++17", "-fPIC",
 # Flags of single sources.  row_kernel.hip: the machine-level loop-invariant code motion would keep
 # literals and addresses of rarely run code (powers, step ends) in some 40 registers across the kernel's
 # loop, which spills the two waves per SIMD that its registers otherwise allow.
-SOURCE_FLAGS = {"row_kernel.hip": ["-mllvm", "-disable-machine-licm"]}
+SOURCE_FLAGS = {"row_kernel.hip": ["-mllvm", "-disable-machine-licm"],
+                "lane_kernel.hip": ["-mllvm", "-disable-machine-licm"]}
 CPP_FLAGS = ["-O2", "-std=c++17", "-fPIC", "-D__HIP_PLATFORM_AMD__", "-I" + os.path.join(ROCM, "include"),
              "-Wall", "-Wno-unused-function"]
 

@@ -529,9 +529,9 @@ struct LaunchShape {
 constexpr int kOrderMinSystems = 16384;
 // Real-only batches of this size or more choose between 16 lanes and one lane per system by trial
 // launches; everything else takes 16 lanes.  One lane per system needs 65,536 systems to give every
-// SIMD one wave and integrates them at the pace of the slowest lane of each wave: 65,536 systems x 365 d
-// take 54.8 ms on it against 18.9 ms on 16 lanes (mixed form), 131,072 67.5 against 37.1 ms, 262,144
-// 65.1 against 73.8 ms, 1,048,576 227 against 294 ms.
+// SIMD one wave and ends at the pace of its slowest lane: 65,536 systems x 365 d take 38.6 ms on it
+// against 18.1 ms on 16 lanes (mixed form), 131,072 53.3 against 35.2 ms, 300,007 53.1 against 80.0 ms,
+// 1,048,576 150 against 277 ms.
 constexpr int kTuneMinSystems = 131072;
 // Systems per trial launch: many resident rounds even at one lane per system, so that every shape is
 // timed at throughput rather than by its slowest systems.
@@ -557,15 +557,23 @@ LaunchShape row_shape(int n) {
     return sh;
 }
 
+// Whether one lane per system means lane_kernel.hip: plain launches of real particles (dense output, the
+// checkpoint features and the extended force model run on the group kernels).
+bool lane_launch(const IntegrateArgs& a, const LaunchShape& sh) {
+    return sh.G == 1 && sh.waves == 1 && a.nvec == 1 && !a.out_t && !ias15_snap(a) && !ext_model(a.fo);
+}
+
 // The integration kernel of a launch shape.
 hipError_t launch_shape(const IntegrateArgs& a, bool mixed, const LaunchShape& sh, int blocks, hipStream_t s,
                         bool set_attributes = true) {
     if (sh.G == kRowLanes) return launch_ias15_row(a, mixed, blocks, sh.threads, s, set_attributes);
+    if (lane_launch(a, sh)) return launch_ias15_lane(a, mixed, blocks, sh.threads, s, set_attributes);
     return launch_ias15(a, sh.G, mixed, sh.waves, blocks, sh.threads, s, set_attributes);
 }
 
 hipError_t shape_occupancy(const IntegrateArgs& a, bool mixed, const LaunchShape& sh, int* blocks_per_cu) {
     if (sh.G == kRowLanes) return ias15_row_occupancy(a, mixed, sh.threads, blocks_per_cu);
+    if (lane_launch(a, sh)) return ias15_lane_occupancy(a, mixed, sh.threads, blocks_per_cu);
     return ias15_occupancy(sh.G, mixed, sh.waves, ext_model(a.fo), ias15_snap(a), a.nvec, sh.threads, blocks_per_cu);
 }
 

@@ -28,6 +28,10 @@ constexpr int kRowLanes = 16, kRowBlock = 256;
 constexpr int kRowTimes = 8, kRowSlice = 88;
 constexpr int kRowWaveWords = 4 * (kRowTimes * kRowSlice + 24);
 
+// The kernel with one lane per system for batches of real particles: words of LDS per lane (the
+// positions of the bodies 1-26 at one time).
+constexpr int kLanePosWords = 3 * 26;
+
 struct ForcesArgs {
     const DevEphem* E;
     ForceOpts fo;
@@ -135,6 +139,11 @@ hipError_t launch_ias15_row(const IntegrateArgs& a, bool mixed, int blocks, int 
                             bool set_attributes = true);
 hipError_t ias15_row_occupancy(const IntegrateArgs& a, bool mixed, int threads, int* blocks_per_cu);
 size_t ias15_row_lds_bytes(int threads);
+// The one-lane kernel of real-only launches (lane_kernel.hip), without checkpoint features, dense output
+// or the extended force model; its scratch is 42 doubles per launched thread.
+hipError_t launch_ias15_lane(const IntegrateArgs& a, bool mixed, int blocks, int threads, hipStream_t s,
+                             bool set_attributes = true);
+hipError_t ias15_lane_occupancy(const IntegrateArgs& a, bool mixed, int threads, int* blocks_per_cu);
 // Whether a launch uses the checkpoint, pause or step-archive features (kernels without them
 // exist for the hot shapes).
 inline bool ias15_snap(const IntegrateArgs& a) { return a.snap_in || a.snap_out || a.t_pause || a.archive; }

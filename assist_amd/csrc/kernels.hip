@@ -1027,8 +1027,6 @@ static const void* ias15_fn() {
 static const void* ias15_lookup(int G, bool mixed, int waves, bool ext, bool snap) {
     if (!snap && !ext && waves == 1) {  // the hot shapes, without the checkpoint features
         switch (G * 2 + (mixed ? 1 : 0)) {
-        case 2: return ias15_fn<1, false, 1, false, false>();
-        case 3: return ias15_fn<1, true, 1, false, false>();
         case 16: return ias15_fn<8, false, 1, false, false>();
         case 17: return ias15_fn<8, true, 1, false, false>();
         default: break;

@@ -1,0 +1,60 @@
+"""The one-lane kernel of real-only launches (lanes_per_system = 1) against the 16-lane kernel that small
+batches run: the same integrator and force model with sums in another order.  Main-belt orbits over at
+most 120 days, where a round-off of 1e-16 grows by less than 1e3 and the mixed form's stop leaves less
+than 1e-11 of a position: 1 m (the 10-year bar of the parity tests) is wide for both, while a wrong
+record, body or substep moves a position by kilometres."""
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+AU_M = 149597870700.0
+
+
+def _both(ephem, t0, t1, states, params=None, **cfg):
+    from assist_amd import batch
+    lane = batch.integrate(ephem, t0, t1, states, params, config=batch.BatchConfig.default(lanes_per_system=1, **cfg))
+    rows = batch.integrate(ephem, t0, t1, states, params, config=batch.BatchConfig.default(**cfg))
+    assert lane.stats.lanes_per_system == 1 and rows.stats.lanes_per_system == 16
+    return lane, rows
+
+
+@pytest.mark.parametrize("precision", [0, 1])
+@pytest.mark.parametrize("marsden", [False, True])
+@pytest.mark.parametrize("n", [1, 63, 65, 1000])
+def test_one_lane_against_rows(gpu, ephem, model, n, marsden, precision):
+    """Both directions, start times over the records of every length (the lanes of a wave are in different
+    ones, and steps cross their ends), and zero-length spans."""
+    from assist_amd import synthetic
+    rng = np.random.default_rng(910 + n)
+    states = np.zeros((n, 1, 6))
+    states[:, 0] = synthetic.main_belt(model, n, rng)
+    params = None
+    if marsden:
+        params = np.zeros((n, 1, 3))
+        params[:, 0] = synthetic.marsden_params(n, rng, 0.5)
+    t0 = rng.uniform(-3000.0, 3000.0, n)
+    t1 = t0 + rng.uniform(-120.0, 120.0, n)
+    t1[:: 7] = t0[:: 7]
+    lane, rows = _both(ephem, t0, t1, states, params, precision=precision)
+    assert (lane.status == 0).all() and (rows.status == 0).all()
+    np.testing.assert_array_equal(lane.states[:: 7], states[:: 7])
+    assert (lane.steps[:: 7] == 0).all()
+    d = np.linalg.norm(lane.states[:, 0, :3] - rows.states[:, 0, :3], axis=-1) * AU_M
+    assert d.max() <= 1.0
+
+
+def test_one_lane_statuses(gpu, ephem, model):
+    """Coverage errors and the step limit end a system and leave the others of its wave alone."""
+    from assist_amd import synthetic
+    n = 130
+    rng = np.random.default_rng(77)
+    states = np.zeros((n, 1, 6))
+    states[:, 0] = synthetic.main_belt(model, n, rng)
+    t0, t1 = np.zeros(n), np.full(n, 100.0)
+    t0[3::5], t1[3::5] = 9.0e4, 9.01e4   # outside the ephemeris from the start
+    lane, rows = _both(ephem, t0, t1, states)
+    np.testing.assert_array_equal(lane.status, rows.status)
+    assert (lane.status[3::5] == 5).all() and (np.delete(lane.status, np.arange(3, n, 5)) == 0).all()
+    lane, rows = _both(ephem, np.zeros(n), np.full(n, 400.0), states, max_steps=20)
+    np.testing.assert_array_equal(lane.status, rows.status)
+    assert (lane.status == -2).all() and (lane.steps == 20).all()
