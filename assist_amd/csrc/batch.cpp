@@ -371,7 +371,9 @@ struct Workspace {
     int device = -1;
     double* scratch = nullptr;
     size_t scratch_words = 0;
-    int* queue = nullptr;
+    int* queue = nullptr;  // the work queue's counter, then the number of late systems
+    double* late = nullptr;
+    size_t late_cap = 0;
     hipEvent_t ev0 = nullptr, ev1 = nullptr, ev_in = nullptr;
     hipStream_t graph_stream = nullptr;  // default priority, non-blocking
     std::vector<GraphEntry> graphs;      // most recently used last
@@ -402,7 +404,7 @@ int ensure_workspace(size_t scratch_words) {
         g_ws.graphs.clear();  // (those of another device are not destroyed from this one)
         g_ws = Workspace();
         g_ws.device = dev;
-        if (!hip_ok(hipMalloc(&g_ws.queue, sizeof(int)), "hipMalloc(queue)")) return ASSIST_BATCH_ERROR_DEVICE;
+        if (!hip_ok(hipMalloc(&g_ws.queue, 2 * sizeof(int)), "hipMalloc(queue)")) return ASSIST_BATCH_ERROR_DEVICE;
         if (!hip_ok(hipEventCreate(&g_ws.ev0), "hipEventCreate") || !hip_ok(hipEventCreate(&g_ws.ev1), "hipEventCreate") ||
             !hip_ok(hipEventCreateWithFlags(&g_ws.ev_in, hipEventDisableTiming), "hipEventCreate") ||
             !hip_ok(hipStreamCreateWithFlags(&g_ws.graph_stream, hipStreamNonBlocking), "hipStreamCreate"))
@@ -416,6 +418,18 @@ int ensure_workspace(size_t scratch_words) {
         if (!hip_ok(hipMalloc(&g_ws.scratch, scratch_words * sizeof(double)), "hipMalloc(scratch)")) return ASSIST_BATCH_ERROR_DEVICE;
         g_ws.scratch_words = scratch_words;
     }
+    return ASSIST_SUCCESS;
+}
+
+// Records of `cap` late systems (the workspace of the current device must exist).
+int ensure_late(size_t cap) {
+    if (cap <= g_ws.late_cap) return ASSIST_SUCCESS;
+    clear_graphs();  // captured launches hold the old pointer
+    (void)hipFree(g_ws.late);
+    g_ws.late = nullptr;
+    g_ws.late_cap = 0;
+    if (!hip_ok(hipMalloc(&g_ws.late, cap * kLateWords * sizeof(double)), "hipMalloc(late)")) return ASSIST_BATCH_ERROR_DEVICE;
+    g_ws.late_cap = cap;
     return ASSIST_SUCCESS;
 }
 
@@ -529,9 +543,10 @@ struct LaunchShape {
 constexpr int kOrderMinSystems = 16384;
 // Real-only batches of this size or more choose between 16 lanes and one lane per system by trial
 // launches; everything else takes 16 lanes.  One lane per system needs 65,536 systems to give every
-// SIMD one wave and ends at the pace of its slowest lane: 65,536 systems x 365 d take 38.6 ms on it
-// against 18.1 ms on 16 lanes (mixed form), 131,072 53.3 against 35.2 ms, 300,007 53.1 against 80.0 ms,
-// 1,048,576 150 against 277 ms.
+// SIMD one wave; its last systems run on 16 lanes (lane_kernel.hip).  On one lane and on 16 (ms): 65,536
+// systems over 365 d 15.9 and 18.1 (mixed form), over 40 d 4.8 and 3.9, over uneven spans up to 10,000 d
+// 188 and 150; 131,072 over 365 d 24.6 and 35.2, over 40 d 6.6 and 7.1; 300,007 over 40 d in double
+// precision 20.9 and 37.5; 1,048,576 over 365 d 151 and 277.
 constexpr int kTuneMinSystems = 131072;
 // Systems per trial launch: many resident rounds even at one lane per system, so that every shape is
 // timed at throughput rather than by its slowest systems.
@@ -577,6 +592,27 @@ hipError_t shape_occupancy(const IntegrateArgs& a, bool mixed, const LaunchShape
     return ias15_occupancy(sh.G, mixed, sh.waves, ext_model(a.fo), ias15_snap(a), a.nvec, sh.threads, blocks_per_cu);
 }
 
+// Block size of the 16-lane kernel on the systems that the one-lane kernel leaves.
+constexpr int kLateThreads = 192;
+
+// Queues an integration: the counters and the kernel and, where a.late is given, the 16-lane kernel for the
+// systems that the one-lane kernel leaves.  `set_attributes`: not while the launches are captured.
+int enqueue_ias15(const IntegrateArgs& a, bool mixed, const LaunchShape& sh, int blocks, int total_groups, hipStream_t s,
+                  bool set_attributes) {
+    if (a.late && !hip_ok(launch_set_counter(a.late_count, 0, s), "launch(set_counter)")) return ASSIST_BATCH_ERROR_DEVICE;
+    if (!hip_ok(launch_set_counter(a.queue, total_groups, s), "launch(set_counter)") ||
+        !hip_ok(launch_shape(a, mixed, sh, blocks, s, set_attributes), "launch(ias15)"))
+        return ASSIST_BATCH_ERROR_DEVICE;
+    if (a.late) {
+        // (the one-lane kernel's grid has one wave per SIMD: as many blocks of three waves fill twice that)
+        const int threads = kLateThreads, late_blocks = std::max(1, 2 * (blocks * sh.threads / 256));
+        if (!hip_ok(launch_set_counter(a.queue, late_blocks * threads / kRowLanes, s), "launch(set_counter)") ||
+            !hip_ok(launch_ias15_row_late(a, mixed, late_blocks, threads, s, set_attributes), "launch(ias15 late)"))
+            return ASSIST_BATCH_ERROR_DEVICE;
+    }
+    return ASSIST_SUCCESS;
+}
+
 // Replays (capturing it first when new) the launch set_counter + ias15_kernel for `a` on the
 // library's graph stream, after the work already queued on `s`; *ms is the graph's HIP-event time.
 int run_ias15_graph(const IntegrateArgs& a, bool mixed, const LaunchShape& sh, int blocks, int total_groups,
@@ -601,8 +637,7 @@ int run_ias15_graph(const IntegrateArgs& a, bool mixed, const LaunchShape& sh, i
         hipGraphExec_t exec = nullptr;
         if (!hip_ok(hipStreamBeginCapture(gs, hipStreamCaptureModeThreadLocal), "hipStreamBeginCapture"))
             return ASSIST_BATCH_ERROR_DEVICE;
-        const bool launched = hip_ok(launch_set_counter(g_ws.queue, total_groups, gs), "launch(set_counter)") &&
-                              hip_ok(launch_shape(a, mixed, sh, blocks, gs, false), "launch(ias15)");
+        const bool launched = enqueue_ias15(a, mixed, sh, blocks, total_groups, gs, false) == ASSIST_SUCCESS;
         const bool captured = hip_ok(hipStreamEndCapture(gs, &graph), "hipStreamEndCapture");
         if (!launched || !captured || !hip_ok(hipGraphInstantiate(&exec, graph, nullptr, nullptr, 0), "hipGraphInstantiate")) {
             if (graph) (void)hipGraphDestroy(graph);
@@ -655,16 +690,25 @@ int run_ias15(IntegrateArgs a, bool mixed, const LaunchShape& sh, int blocks_per
     a.scratch = g_ws.scratch;
     a.ecache = cw ? g_ws.scratch + (size_t)blocks * sh.threads * 42 : nullptr;
     a.queue = g_ws.queue;
+    if (lane_launch(a, sh) && a.nsys >= kTuneMinSystems) {
+        const int cap = blocks * sh.threads / 64 * kLateLanes;
+        rc = ensure_late((size_t)cap);
+        if (rc) return rc;
+        if (!hip_ok(ias15_row_occupancy(a, mixed, kLateThreads, &per_cu, true), "occupancy")) return ASSIST_BATCH_ERROR_DEVICE;
+        a.late = g_ws.late;
+        a.late_cap = cap;
+        a.late_count = g_ws.queue + 1;
+    }
     if (use_graph) {
         rc = run_ias15_graph(a, mixed, sh, blocks, total_groups, s, ms);
         if (rc) return rc;
         if (blocks_out) *blocks_out = blocks;
         return ASSIST_SUCCESS;
     }
-    if (!hip_ok(launch_set_counter(g_ws.queue, total_groups, s), "launch(set_counter)") ||
-        !hip_ok(hipEventRecord(g_ws.ev0, s), "hipEventRecord") ||
-        !hip_ok(launch_shape(a, mixed, sh, blocks, s), "launch(ias15)") ||
-        !hip_ok(hipEventRecord(g_ws.ev1, s), "hipEventRecord") || !hip_ok(hipEventSynchronize(g_ws.ev1), "ias15"))
+    if (!hip_ok(hipEventRecord(g_ws.ev0, s), "hipEventRecord")) return ASSIST_BATCH_ERROR_DEVICE;
+    rc = enqueue_ias15(a, mixed, sh, blocks, total_groups, s, true);
+    if (rc) return rc;
+    if (!hip_ok(hipEventRecord(g_ws.ev1, s), "hipEventRecord") || !hip_ok(hipEventSynchronize(g_ws.ev1), "ias15"))
         return ASSIST_BATCH_ERROR_DEVICE;
     float t = 0.f;
     (void)hipEventElapsedTime(&t, g_ws.ev0, g_ws.ev1);

@@ -94,8 +94,19 @@ struct IntegrateArgs {
     double* archive;
     int* archive_count;
     int archive_cap;
-    int pad2_;
+    // systems that the one-lane kernel leaves to the 16-lane kernel (optional): up to late_cap records of
+    // kLateWords doubles and their number
+    int late_cap;
+    double* late;
+    int* late_count;
 };
+
+// Record of a system at a step boundary: its index, t, the next trial step, the last accepted step, steps,
+// evaluations, rejections, a pad word, x, v and their Kahan compensations (3 each), then the last step's b
+// and the correction e of its prediction (21 each, k-major), padded to 64.
+constexpr int kLateWords = 64;
+// A wave of the one-lane kernel whose systems have run out leaves its last ones when this many are left.
+constexpr int kLateLanes = 32;
 
 // Doubles of the substep ephemeris cache per launched thread (0 when the kernel keeps none):
 // 8-lane groups outside the extended model keep 88 words per substep and group.  (One lane per
@@ -137,7 +148,10 @@ hipError_t ias15_occupancy(int G, bool mixed, int waves, bool ext, bool snap, in
 // force model; its scratch is 28 doubles per launched thread at most.
 hipError_t launch_ias15_row(const IntegrateArgs& a, bool mixed, int blocks, int threads, hipStream_t s,
                             bool set_attributes = true);
-hipError_t ias15_row_occupancy(const IntegrateArgs& a, bool mixed, int threads, int* blocks_per_cu);
+// The same for the systems of a.late (its queue starts at the grid's rows).
+hipError_t launch_ias15_row_late(const IntegrateArgs& a, bool mixed, int blocks, int threads, hipStream_t s,
+                                 bool set_attributes = true);
+hipError_t ias15_row_occupancy(const IntegrateArgs& a, bool mixed, int threads, int* blocks_per_cu, bool late = false);
 size_t ias15_row_lds_bytes(int threads);
 // The one-lane kernel of real-only launches (lane_kernel.hip), without checkpoint features, dense output
 // or the extended force model; its scratch is 42 doubles per launched thread.

@@ -19,10 +19,18 @@
 //   * without variational vectors no partials are compiled in, and without Marsden parameters not that
 //     term either.
 //
+// A wave runs for as long as one of its lanes does, and a trip takes as long with one active lane as with
+// 64.  In large batches a wave whose list of systems has run out therefore leaves its last ones (at most
+// kLateLanes) at a step boundary to the 16-lane kernel, which takes them on from there at a tenth of the
+// time per evaluation.  Each wave has its own list, so which systems these are, and every result, is the
+// same in every run.  (With 32 of 64 lanes left a wave's rate falls to the 16-lane kernel's; 48 and 20
+// took 2% and up to 18% longer.)
+//
 // What bounds it: the L1 look-ups (1.3 a clock), then the latency of a wave's own loads (25% of its
 // cycles; vector instructions issue in 40%).  Measured on an MI355X against one time per trip:
 // 1,048,576 systems over 365 d 221 -> 149 ms in the mixed form from the learned start, 493 -> 330 ms in
-// double precision.
+// double precision; with the last systems left to the 16-lane kernel 300,007 systems over 40 d 28.3 -> 20.9 ms
+// (double precision, 37.4 on 16 lanes alone), 131,072 over 365 d 53.3 -> 24.6 ms (mixed, 35.2).
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
@@ -325,8 +333,13 @@ ias15_lane_kernel(IntegrateArgs args) {
     // attempt), or neither (a repeated pass)
     bool start = true, predict = true;
     bool ng = false;
-    bool active = tid < ka->nsys;
-    int sys = active ? (ka->order ? ka->order[tid] : tid) : 0;
+    // a wave's systems are the positions wave, wave + nwaves, wave + 2 nwaves, ... of the order: which
+    // systems it leaves to the 16-lane kernel does not depend on the other waves' pace
+    const int nwaves = (int)((gridDim.x * blockDim.x) >> 6), wave = tid >> 6;
+    auto position = [&](int k) { return (long long)k * nwaves + wave; };
+    int taken = 64;  // (the same on all active lanes)
+    bool active = position(wl) < ka->nsys;
+    int sys = active ? (ka->order ? ka->order[position(wl)] : (int)position(wl)) : 0;
 
     auto load = [&](int s) {
         const double* st = ka->states + (size_t)s * 6;
@@ -367,12 +380,43 @@ ias15_lane_kernel(IntegrateArgs args) {
         if (ka->evals) ka->evals[sys] = evals;
         if (ka->rejected) ka->rejected[sys] = rejected;
         if (ka->t_out) ka->t_out[sys] = t;
-        const int next = atomicAdd(ka->queue, 1);
-        active = next < ka->nsys;
-        if (active) {
-            sys = ka->order ? ka->order[next] : next;
-            load(sys);
+    };
+    // Lanes that are done write their system and take the wave's next ones, in the order of the lanes; all
+    // active lanes call this together.  (A system with a zero-length span is done at once.)
+    auto take_next = [&](bool done) {
+#if defined(__HIP_DEVICE_COMPILE__)
+        for (unsigned long long fin = __ballot(done); fin != 0ULL; fin = __ballot(done)) {
+            if (done) {
+                finish();
+                const int k = taken + (int)__builtin_amdgcn_mbcnt_hi((unsigned)(fin >> 32),
+                                                                     __builtin_amdgcn_mbcnt_lo((unsigned)fin, 0u));
+                const long long q = position(k);
+                active = q < ka->nsys;
+                done = false;
+                if (active) {
+                    sys = ka->order ? ka->order[q] : (int)q;
+                    load(sys);
+                    done = t == t_end;
+                }
+            }
+            taken += (int)__popcll(fin);
         }
+#endif
+    };
+    // Leaves the system, at a step boundary, to the 16-lane kernel.
+    auto leave = [&]() {
+        const int q = atomicAdd(ka->late_count, 1);
+        if (q >= ka->late_cap) return;  // (it stays here)
+        double* const rec = ka->late + (size_t)q * kLateWords;
+        const double* const scr = scratch();
+        rec[0] = (double)sys; rec[1] = t; rec[2] = dt; rec[3] = dt_last;
+        rec[4] = (double)steps; rec[5] = (double)evals; rec[6] = (double)rejected;
+#pragma unroll
+        for (int c = 0; c < 3; c++) { rec[8 + c] = x0[c]; rec[11 + c] = v0[c]; rec[14 + c] = csx[c]; rec[17 + c] = csv[c]; }
+        const bool stepped = dt_last != 0.0;
+#pragma unroll 6
+        for (int k = 0; k < 42; k++) rec[20 + k] = stepped ? scr[k * 64] : 0.0;
+        active = false;
     };
     // Predict b of the attempt from the last accepted step and convert it to g.
     auto setup_attempt = [&]() {
@@ -448,7 +492,7 @@ ias15_lane_kernel(IntegrateArgs args) {
 
     if (active) {
         load(sys);
-        while (active && t == t_end) finish();  // (zero-length spans)
+        take_next(t == t_end);
     }
     while (active) {
         ka = launder(ka);
@@ -565,8 +609,9 @@ ias15_lane_kernel(IntegrateArgs args) {
             else if (p == 2) correct<5>(at, a0, b, g, tmp);
             else correct<7>(at, a0, b, g, tmp);
         }
-        bool done = status != 0;
-        if (!done) {
+        // (returns whether the system is done)
+        auto end_pass = [&]() -> bool {
+            if (status != 0) return true;
             // ---- end of a predictor-corrector iteration (the tests are ias15_kernel's) ----
             double maxak = 0.0, maxdb6 = 0.0;
 #pragma unroll
@@ -584,7 +629,7 @@ ias15_lane_kernel(IntegrateArgs args) {
                 !(it > 2 && pc_err_last <= pc_err) && it < 12) {
                 pc_err_last = pc_err;
                 it++;
-                continue;
+                return false;
             }
             // ---- step-size control ----
             double dt_new = dts, dt_prop = dts;
@@ -604,7 +649,7 @@ ias15_lane_kernel(IntegrateArgs args) {
                     dts = dt_new;
                     last = 0;
                     predict = true;
-                    continue;
+                    return false;
                 }
                 dt_prop = dt_new;
                 if (dt_new / dts > 1. / 0.25) dt_new = dts / 0.25;
@@ -666,14 +711,14 @@ ias15_lane_kernel(IntegrateArgs args) {
             dt_last = dts;
             if (!(last && ka->io.epsilon <= 0)) dt = dt_new;
             start = predict = true;
-            if (bad) { status = kNonFinite; done = true; }
-            else if (last) done = true;
-            else if (steps >= ka->io.max_steps) { status = kMaxSteps; done = true; }
-        }
-        if (done) {
-            do finish();
-            while (active && t == t_end);
-        }
+            if (bad) { status = kNonFinite; return true; }
+            if (last) return true;
+            if (steps >= ka->io.max_steps) { status = kMaxSteps; return true; }
+            return false;
+        };
+        take_next(end_pass());
+        // (lanes run out only when the wave's systems have)
+        if (ka->late && (int)__popcll(__ballot(active)) <= kLateLanes && active && start) leave();
     }
 }
 

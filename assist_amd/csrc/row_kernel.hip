@@ -388,7 +388,8 @@ constexpr int kRowAlign = 2;
 
 // NV: vectors per lane quad (1: up to 4 vectors per system, 2: up to 8).  Jacobian: the systems
 // carry variational vectors.
-template <bool Mixed, int NV, bool Jacobian, int Model>
+// Late: the systems are the records that the one-lane kernel left (a.late).
+template <bool Mixed, int NV, bool Jacobian, int Model, bool Late = false>
 __global__ void __launch_bounds__(kRowBlock) __attribute__((amdgpu_waves_per_eu(row_waves(Mixed, Jacobian, Model), row_waves(Mixed, Jacobian, Model))))
 ias15_row_kernel(IntegrateArgs args) {
     (void)args;
@@ -459,8 +460,10 @@ ias15_row_kernel(IntegrateArgs args) {
     // spreads over every wave
     const int nwaves = (int)((gridDim.x * blockDim.x) >> 6);
     const int q0 = row * nwaves + wave;
-    bool active = q0 < ka->nsys;
-    int sys = active ? (ka->order ? ka->order[q0] : q0) : 0;
+    auto systems = [&]() { return Late ? min(*ka->late_count, ka->late_cap) : ka->nsys; };
+    auto system_at = [&](int q) { return Late ? (int)ka->late[(size_t)q * kLateWords] : (ka->order ? ka->order[q] : q); };
+    bool active = q0 < systems();
+    int sys = active ? system_at(q0) : 0;
 
     auto load = [&](int s) {
         const double* st = ka->states + (size_t)s * nv * 6;
@@ -516,6 +519,26 @@ ias15_row_kernel(IntegrateArgs args) {
         steps = evals = rejected = 0;
         last = 0;
     };
+    // a system that the one-lane kernel left, at the step boundary of its record
+    auto resume = [&](int q) {
+        const double* const rec = ka->late + (size_t)q * kLateWords;
+        const double tr = rec[1], dtr = rec[2], dlr = rec[3], st = rec[4], ev = rec[5], rj = rec[6];
+        if (own[0]) {
+            x0[0] = rec[8 + c];
+            v0[0] = rec[11 + c];
+            csx[0] = rec[14 + c];
+            csv[0] = rec[17 + c];
+        }
+        double* const scr = scratch();
+#pragma unroll
+        for (int k = 0; k < 14; k++) scr[k * 64] = rec[20 + 3 * k + c];
+        t = tr;
+        dt = dtr;
+        dt_last = dlr;
+        steps = (long long)st;
+        evals = (long long)ev;
+        rejected = (long long)rj;
+    };
     auto finish = [&]() {
         double* st = ka->states + (size_t)sys * nv * 6;
 #pragma unroll
@@ -536,10 +559,11 @@ ias15_row_kernel(IntegrateArgs args) {
             next = atomicAdd(ka->queue, 1);
         }
         next = row_bcast0_i(next);
-        active = next < ka->nsys;
+        active = next < systems();
         if (active) {
-            sys = ka->order ? ka->order[next] : next;
+            sys = system_at(next);
             load(sys);
+            if constexpr (Late) resume(next);
         }
     };
     // Predict b of the attempt from the last accepted step and convert it to g.  Returns false
@@ -599,7 +623,10 @@ ias15_row_kernel(IntegrateArgs args) {
         return true;
     };
 
-    if (active) load(sys);
+    if (active) {
+        load(sys);
+        if constexpr (Late) resume(q0);
+    }
     if (!active) need_eph = false;
     // A row whose queue ran dry stays in the loop while any row of its wave is active: all 64 lanes
     // take part in the ephemeris rounds.
@@ -901,19 +928,20 @@ ias15_row_kernel(IntegrateArgs args) {
     }
 }
 
-template <bool M, int NV, bool J>
+template <bool M, int NV, bool J, bool Late = false>
 static const void* row_fn(int model) {
     if constexpr (!M) {
-        if (model == kModelStd) return (const void*)ias15_row_kernel<M, NV, J, kModelStd>;
+        if (model == kModelStd) return (const void*)ias15_row_kernel<M, NV, J, kModelStd, Late>;
     }
-    return model == kModelGravity ? (const void*)ias15_row_kernel<M, NV, J, kModelGravity>
-                                  : (const void*)ias15_row_kernel<M, NV, J, kModelAny>;
+    return model == kModelGravity ? (const void*)ias15_row_kernel<M, NV, J, kModelGravity, Late>
+                                  : (const void*)ias15_row_kernel<M, NV, J, kModelAny, Late>;
 }
 
-static const void* row_lookup(const IntegrateArgs& a, bool mixed) {
+static const void* row_lookup(const IntegrateArgs& a, bool mixed, bool late = false) {
     const bool std_forces = a.fo.forces == kStdForces && a.fo.gr_eih_sources > 0;
     int m = kModelAny;
     if (mixed || std_forces) m = !a.params ? kModelGravity : (mixed ? kModelAny : kModelStd);
+    if (late) return a.nvec != 1 ? nullptr : (mixed ? row_fn<true, 1, false, true>(m) : row_fn<false, 1, false, true>(m));
     if (a.nvec == 1) return mixed ? row_fn<true, 1, false>(m) : row_fn<false, 1, false>(m);
     if (a.nvec <= 4) return mixed ? row_fn<true, 1, true>(m) : row_fn<false, 1, true>(m);
     if (a.nvec <= 8) return mixed ? row_fn<true, 2, true>(m) : row_fn<false, 2, true>(m);
@@ -924,8 +952,7 @@ size_t ias15_row_lds_bytes(int threads) {
     return (kTabWords + (size_t)(threads / 64) * kRowWaveWords) * sizeof(double);
 }
 
-hipError_t launch_ias15_row(const IntegrateArgs& a, bool mixed, int blocks, int threads, hipStream_t s, bool set_attributes) {
-    const void* f = row_lookup(a, mixed);
+static hipError_t launch_row(const void* f, const IntegrateArgs& a, int blocks, int threads, hipStream_t s, bool set_attributes) {
     if (!f || threads % 64 != 0 || threads > kRowBlock) return hipErrorInvalidValue;
     const size_t lds = ias15_row_lds_bytes(threads);
     hipError_t e = hipSuccess;
@@ -939,8 +966,16 @@ hipError_t launch_ias15_row(const IntegrateArgs& a, bool mixed, int blocks, int 
     return hipGetLastError();
 }
 
-hipError_t ias15_row_occupancy(const IntegrateArgs& a, bool mixed, int threads, int* blocks_per_cu) {
-    const void* f = row_lookup(a, mixed);
+hipError_t launch_ias15_row(const IntegrateArgs& a, bool mixed, int blocks, int threads, hipStream_t s, bool set_attributes) {
+    return launch_row(row_lookup(a, mixed), a, blocks, threads, s, set_attributes);
+}
+
+hipError_t launch_ias15_row_late(const IntegrateArgs& a, bool mixed, int blocks, int threads, hipStream_t s, bool set_attributes) {
+    return launch_row(row_lookup(a, mixed, true), a, blocks, threads, s, set_attributes);
+}
+
+hipError_t ias15_row_occupancy(const IntegrateArgs& a, bool mixed, int threads, int* blocks_per_cu, bool late) {
+    const void* f = row_lookup(a, mixed, late);
     if (!f) return hipErrorInvalidValue;
     const size_t lds = ias15_row_lds_bytes(threads);
     hipError_t e = hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);

@@ -58,3 +58,40 @@ def test_one_lane_statuses(gpu, ephem, model):
     lane, rows = _both(ephem, np.zeros(n), np.full(n, 400.0), states, max_steps=20)
     np.testing.assert_array_equal(lane.status, rows.status)
     assert (lane.status == -2).all() and (lane.steps == 20).all()
+
+
+@pytest.mark.parametrize("precision", [0, 1])
+@pytest.mark.parametrize("marsden", [False, True])
+def test_last_systems_of_a_large_batch(gpu, ephem, model, marsden, precision):
+    """In a batch of 131,072 systems or more every wave leaves its last systems to the 16-lane kernel: the
+    same systems in batches below that stay on one lane throughout.  Lists of 128 and 129 systems a wave,
+    zero-length spans and systems outside the ephemeris among them; twice the same bits."""
+    from assist_amd import batch, synthetic
+    n = 131072 + 65
+    rng = np.random.default_rng(5)
+    states = np.zeros((n, 1, 6))
+    states[:, 0] = synthetic.main_belt(model, n, rng)
+    params = None
+    if marsden:
+        params = np.zeros((n, 1, 3))
+        params[:, 0] = synthetic.marsden_params(n, rng, 0.5)
+    t0 = rng.uniform(-3000.0, 3000.0, n)
+    t1 = t0 + rng.uniform(-60.0, 60.0, n)
+    t1[::11] = t0[::11]
+    t0[5::1001], t1[5::1001] = 9.0e4, 9.01e4
+    cfg = batch.BatchConfig.default(lanes_per_system=1, precision=precision)
+    whole = batch.integrate(ephem, t0, t1, states, params, config=cfg)
+    again = batch.integrate(ephem, t0, t1, states, params, config=cfg)
+    for k in ("states", "status", "steps"):
+        np.testing.assert_array_equal(getattr(whole, k), getattr(again, k))
+    h = n // 2
+    parts = [batch.integrate(ephem, t0[s], t1[s], states[s], None if params is None else params[s], config=cfg)
+             for s in (slice(0, h), slice(h, n))]
+    np.testing.assert_array_equal(whole.status, np.concatenate([p.status for p in parts]))
+    assert (whole.status[5::1001] == 5).all() and (whole.status == 5).sum() == len(t0[5::1001])
+    ok = whole.status == 0
+    d = np.linalg.norm(whole.states[:, 0, :3] - np.concatenate([p.states for p in parts])[:, 0, :3], axis=-1) * AU_M
+    assert d[ok].max() <= 1.0
+    # a step's length is the seventh root of its error estimate: round-off moves few step counts
+    steps = np.concatenate([p.steps for p in parts])
+    assert (np.abs(whole.steps - steps) <= 1).mean() > 0.999 and abs(whole.stats.steps - steps.sum()) < 1e-3 * steps.sum()
