@@ -95,3 +95,30 @@ def test_last_systems_of_a_large_batch(gpu, ephem, model, marsden, precision):
     # a step's length is the seventh root of its error estimate: round-off moves few step counts
     steps = np.concatenate([p.steps for p in parts])
     assert (np.abs(whole.steps - steps) <= 1).mean() > 0.999 and abs(whole.stats.steps - steps.sum()) < 1e-3 * steps.sum()
+
+
+def test_large_batch_in_a_graph(gpu, ephem, model):
+    """The captured launches of a large batch (counters, one-lane kernel, 16-lane kernel for the systems it
+    leaves): every replay gives the eager launch's bits, with other work between them."""
+    from assist_amd import batch, synthetic
+    n = 131072 + 65
+    rng = np.random.default_rng(8)
+    states = np.zeros((n, 1, 6))
+    states[:, 0] = synthetic.main_belt(model, n, rng)
+    t0, t1 = rng.uniform(-2000.0, 2000.0, n), np.zeros(n)
+    t1[:] = t0 + rng.uniform(-40.0, 40.0, n)
+    d0, d1, first = batch.DeviceArray(t0), batch.DeviceArray(t1), batch.DeviceArray(states)
+    st, status = batch.DeviceArray(states), batch.DeviceArray(np.zeros(n, np.int32))
+
+    def run(**cfg):
+        st.copy_from(first)
+        batch.integrate_device(ephem, n, 0, d0, d1, st, None, status, None, None,
+                               config=batch.BatchConfig.default(lanes_per_system=1, precision=1, **cfg))
+        return st.download()
+
+    eager = run()
+    assert (status.download() == 0).all()
+    for _ in range(3):
+        np.testing.assert_array_equal(run(use_graph=1), eager)
+        batch.synchronize()
+        np.testing.assert_array_equal(run(), eager)
