@@ -572,6 +572,50 @@ LaunchShape row_shape(int n) {
     return sh;
 }
 
+// Block size of the group kernels: batches too small to give every CU a 256-thread block take 128-thread
+// blocks, so that their waves spread over all CUs (configuration 2: 3% faster).
+int group_block(int n, int G) {
+    int dev = 0, ncu = 0;
+    if (hip_ok(hipGetDevice(&dev), "hipGetDevice") &&
+        hip_ok(hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, dev), "hipDeviceGetAttribute") &&
+        (long long)n * G < (long long)kIas15Block * ncu)
+        return 128;
+    return kIas15Block;
+}
+
+// Checkpoint, pause and archive launches of real particles run on ias15_kernel, on 8 lanes per system or on
+// one.  One lane does about a third of the work per evaluation, but its launch lasts as long as its costliest
+// system, which a lane integrates 2.5 times slower than 8 lanes do: it wins where the batch keeps 65,536
+// lanes busy for longer than that.  With the steps that a system takes (about 7 + 0.15 |t1 - t0| / q, the
+// fit behind the queue order) the line is sum of the steps = kOneLaneShare x the costliest system's.
+// Eight lanes' time over one lane's, in double precision and in the mixed form, at that share: 26,000
+// (131,072 systems, spans from 30 to 365 d) 0.69, 0.92; 33,000 (131,072 over 365 d) 0.90, 1.14; 39,000
+// (180,001, 30 to 365 d) 0.80, 1.24; 44,000 (262,144, 30 to 365 d) 1.17, 1.30; 45,000 (180,001 over 365 d)
+// 1.30, 1.73; 106,000 (131,072 over 5 d) 2.5, 2.7; 262,000 (1,048,576 over 365 d) 2.0, 2.4.
+constexpr double kOneLaneShare = 42000.0;
+constexpr int kShareSample = 1024;  // systems of the sorted queue that stand for all
+
+// Whether the batch's n sorted queue keys (device; launch_span_order) put it on one lane.
+int one_lane_share(const unsigned long long* keys, int n, hipStream_t s, bool* one) {
+    const int m = std::min(n, kShareSample);
+    const size_t stride = (size_t)(n / m) * sizeof *keys;
+    unsigned long long h[kShareSample];
+    if (!hip_ok(hipMemcpy2DAsync(h, sizeof *h, keys, stride, sizeof *h, (size_t)m, hipMemcpyDeviceToHost, s), "hipMemcpy2DAsync") ||
+        !hip_ok(hipStreamSynchronize(s), "queue order"))
+        return ASSIST_BATCH_ERROR_DEVICE;
+    double sum = 0.0, most = 0.0;
+    for (int i = 0; i < m; i++) {
+        const unsigned long long bits = h[i] & ~kKeyRateMask;
+        double span;
+        memcpy(&span, &bits, sizeof span);
+        const double steps = 7.0 + 0.15e-3 * span * (double)(h[i] & kKeyRateMask);
+        sum += steps;
+        most = std::max(most, steps);
+    }
+    *one = sum < 1e300 && (double)n / m * sum >= kOneLaneShare * most;
+    return ASSIST_SUCCESS;
+}
+
 // Whether one lane per system means lane_kernel.hip: plain launches of real particles (dense output, the
 // checkpoint features and the extended force model run on the group kernels).
 bool lane_launch(const IntegrateArgs& a, const LaunchShape& sh) {
@@ -1024,16 +1068,7 @@ static int integrate_device_locked(const struct assist_ephem* ephem, const struc
     }
     shape.G = lanes_for(nv, lanes_req);
     if (shape.G < 0) return ASSIST_BATCH_ERROR_ARG;
-    shape.threads = cfg.block_size > 0 ? cfg.block_size : kIas15Block;
-    if (cfg.block_size == 0 && shape.G > 0) {
-        // untuned batches too small to give every CU a 256-thread block take 128-thread blocks,
-        // so that their waves spread over all CUs (configuration 2: 3% faster)
-        int dev = 0, ncu = 0;
-        if (hip_ok(hipGetDevice(&dev), "hipGetDevice") &&
-            hip_ok(hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, dev), "hipDeviceGetAttribute") &&
-            (long long)n * shape.G < (long long)kIas15Block * ncu)
-            shape.threads = 128;
-    }
+    shape.threads = cfg.block_size > 0 ? cfg.block_size : group_block(n, shape.G);
     if (shape.threads % 64 != 0 || shape.threads > kIas15Block || shape.threads % shape.G != 0) return ASSIST_BATCH_ERROR_ARG;
     shape.waves = cfg.waves_per_simd > 0 ? cfg.waves_per_simd : 1;
     if (shape.waves != 1 && shape.waves != 2) return ASSIST_BATCH_ERROR_ARG;
@@ -1041,7 +1076,7 @@ static int integrate_device_locked(const struct assist_ephem* ephem, const struc
     const bool ext = ext_model(a.fo);
     if (ext && (mixed || shape.waves != 1)) return ASSIST_BATCH_ERROR_UNSUPPORTED;
     // with no launch override: 16 lanes per system, or one (the checkpoint features and the extended
-    // force model run on the group kernels alone)
+    // force model run on the group kernels alone, on 8 lanes or, below, on one)
     const bool choose = lanes_req == 0 && cfg.block_size == 0 && cfg.waves_per_simd == 0 && !ext && !ias15_snap(a);
     if (choose) shape = row_shape(n);
     // the substep cache pays when attempts take several passes: by default it is off with the
@@ -1063,6 +1098,16 @@ static int integrate_device_locked(const struct assist_ephem* ephem, const struc
                     "launch(queue order)"))
             return ASSIST_BATCH_ERROR_DEVICE;
         a.order = g_ws.order;
+        // (a resumed batch keeps its snapshots' lanes)
+        if (ias15_snap(a) && nv == 1 && lanes_req == 0 && cfg.block_size == 0 && cfg.waves_per_simd == 0 && !ext) {
+            bool one = false;
+            rc = one_lane_share(g_ws.okeys_alt, n, s, &one);
+            if (rc) return rc;
+            if (one) {
+                shape.G = 1;
+                shape.threads = group_block(n, 1);
+            }
+        }
     }
     float ms = 0.f;
     int blocks = 0;

@@ -175,7 +175,10 @@ constexpr int kNoAllocMaxDevices = 64;
 hipError_t noalloc_scratch(double** ptr);
 // Queue order of large batches: order[0..n) = system indices sorted by span |t1 - t0|, longest
 // first, and among equal spans by the real particle's perihelion distance, smallest first (stable,
-// so equal keys keep their index order).  Buffers: keys/keys_alt n words, vals n ints.
+// so equal keys keep their index order).  Buffers: keys/keys_alt n words, vals n ints; keys_alt
+// receives the sorted keys: the span's bit pattern with the bits of kKeyRateMask replaced by
+// 1000 / q (q in au; 0 for a span that is no number).
+constexpr unsigned long long kKeyRateMask = 0xFFFFFull;
 size_t span_order_temp_bytes(int n);
 hipError_t launch_span_order(const DevEphem* E, int n, int nvec, const double* t0, const double* t1,
                              const double* states, unsigned long long* keys, unsigned long long* keys_alt, int* vals,

@@ -935,8 +935,8 @@ hipError_t launch_archive_interp(int nsys, int nq, int nvec, int cap, const doub
 // main-belt and NEO-like orbits (a fit over 800-10 000-day spans, 11% rms in log), but a close
 // approach can multiply that, so the longest spans go first whatever their orbits, and among
 // equal spans the smallest perihelia.  The key is the span's bit pattern with its low 20 bits
-// (below 2^-32 of the span) replaced by min(1/q, 1000) x 1000.  Only the order of the queue
-// depends on the key.
+// (below 2^-32 of the span) replaced by min(1/q, 1000) x 1000.  The order of the
+// queue depends on the key, and the lanes per system of checkpoint launches.
 __global__ void span_keys_kernel(const DevEphem* __restrict__ E, int n, int nvec, const double* __restrict__ t0,
                                  const double* __restrict__ t1, const double* __restrict__ states,
                                  unsigned long long* __restrict__ keys, int* __restrict__ vals) {
@@ -959,7 +959,7 @@ __global__ void span_keys_kernel(const DevEphem* __restrict__ E, int n, int nvec
     const double rate = (q == q) ? fmin(1.0 / fmax(q, 1e-3), 1000.0) : 0.0;
     const unsigned long long low = (unsigned long long)(rate * 1000.0);  // < 2^20
     // non-negative doubles sort like their bit patterns; NaN sorts last
-    keys[i] = (span == span) ? (((unsigned long long)__double_as_longlong(span) & ~0xFFFFFull) | low) : 0ull;
+    keys[i] = (span == span) ? (((unsigned long long)__double_as_longlong(span) & ~kKeyRateMask) | low) : 0ull;
     vals[i] = i;
 }
 
