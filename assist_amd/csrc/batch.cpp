@@ -7,9 +7,7 @@
 #include <string.h>
 
 #include <algorithm>
-#include <map>
 #include <mutex>
-#include <tuple>
 #include <vector>
 
 #include "../../include/ascii_ephem.h"
@@ -525,11 +523,11 @@ void pack(const reb_simulation* sim, const assist_extras* ax, const SimLayout& L
 
 }  // namespace
 
-// ---- launch of the integration kernel and its autotuner ----------------------------------
+// ---- launch of the integration kernel -------------------------------------------------------
 namespace {
 
-// The workspace, the graph cache and the tuner's choices are process-wide: the integration entry
-// points hold this lock from the shape choice to the kernel's completion, so that calls from
+// The workspace and the graph cache are process-wide: the integration entry points hold this lock
+// from the shape choice to the kernel's completion, so that calls from
 // several host threads run one after another instead of sharing one work queue and scratch.
 std::mutex g_launch_mutex;
 
@@ -541,17 +539,17 @@ struct LaunchShape {
 
 // Batches of this size or more hand out their systems in the queue order.
 constexpr int kOrderMinSystems = 16384;
-// Real-only batches of this size or more choose between 16 lanes and one lane per system by trial
-// launches; everything else takes 16 lanes.  One lane per system needs 65,536 systems to give every
-// SIMD one wave; its last systems run on 16 lanes (lane_kernel.hip).  On one lane and on 16 (ms): 65,536
-// systems over 365 d 15.9 and 18.1 (mixed form), over 40 d 4.8 and 3.9, over uneven spans up to 10,000 d
-// 188 and 150; 131,072 over 365 d 24.6 and 35.2, over 40 d 6.6 and 7.1; 300,007 over 40 d in double
-// precision 20.9 and 37.5; 1,048,576 over 365 d 151 and 277.
-constexpr int kTuneMinSystems = 131072;
-// Systems per trial launch: many resident rounds even at one lane per system, so that every shape is
-// timed at throughput rather than by its slowest systems.
-constexpr int kTuneSample = 1048576;
-constexpr double kTuneSpan = 30.0;      // days integrated per trial system
+// Real-only batches of this size or more take one lane per system, everything else 16.  The line is a
+// number of systems alone: the two kernels sum in another order, and results must not depend on which of
+// them a timing prefers.  One lane per system needs 65,536 systems to give every SIMD one wave; its last
+// systems run on 16 lanes (lane_kernel.hip).  On one lane and on 16 (ms, mixed form): 65,536 systems over
+// 365 d 15.9 and 18.1, over 40 d 4.8 and 3.9, over uneven spans up to 10,000 d 188 and 150.  In double
+// precision and in the mixed form: 131,072 over 1 d 4.4 and 8.9, 4.6 and 8.3; over 40 d 12.0 and 16.5, 9.0
+// and 13.1; over 365 d 49.6 and 63.4, 26.9 and 41.4; over uneven spans from 30 to 3,000 d 143 and 112, 75
+// and 67; 262,144 over those 218 and 208, 107 and 133; over 365 d 87 and 126, 44 and 82; 1,048,576 over
+// 365 d 333 and 498, 165 and 325.  (Blocks of 128 threads, of which a CU's LDS holds one, took 1.2 to 1.9
+// times as long as blocks of 256 at every size.)
+constexpr int kLaneMinSystems = 131072;
 
 // The shape of the 16-lane kernel for n systems.  A trip of a wave takes as long with one system as
 // with four, so systems go one to a wave while every SIMD has room for another wave (blocks of one
@@ -734,7 +732,7 @@ int run_ias15(IntegrateArgs a, bool mixed, const LaunchShape& sh, int blocks_per
     a.scratch = g_ws.scratch;
     a.ecache = cw ? g_ws.scratch + (size_t)blocks * sh.threads * 42 : nullptr;
     a.queue = g_ws.queue;
-    if (lane_launch(a, sh) && a.nsys >= kTuneMinSystems) {
+    if (lane_launch(a, sh) && a.nsys >= kLaneMinSystems) {
         const int cap = blocks * sh.threads / 64 * kLateLanes;
         rc = ensure_late((size_t)cap);
         if (rc) return rc;
@@ -758,88 +756,6 @@ int run_ias15(IntegrateArgs a, bool mixed, const LaunchShape& sh, int blocks_per
     (void)hipEventElapsedTime(&t, g_ws.ev0, g_ws.ev1);
     if (ms) *ms = t;
     if (blocks_out) *blocks_out = blocks;
-    return ASSIST_SUCCESS;
-}
-
-struct TuneKey {
-    int dev, size, mixed, forces, has_params;  // size: the systems' power of two
-    bool operator<(const TuneKey& o) const {
-        return std::tie(dev, size, mixed, forces, has_params) <
-               std::tie(o.dev, o.size, o.mixed, o.forces, o.has_params);
-    }
-};
-std::map<TuneKey, LaunchShape> g_tuned;
-
-// Picks the kernel and block size for a real-only batch by timing each candidate on copies of its
-// first kTuneSample systems over at most kTuneSpan days (the caller's buffers are not touched); the
-// choice is cached per device, configuration and size class.
-int tuned_shape(const IntegrateArgs& base, bool mixed, hipStream_t s, LaunchShape* out) {
-    int dev = 0;
-    if (!hip_ok(hipGetDevice(&dev), "hipGetDevice")) return ASSIST_BATCH_ERROR_DEVICE;
-    int size = 0;
-    while (size < 30 && (base.nsys >> (size + 1)) > 0) size++;
-    const TuneKey key{dev, size, mixed ? 1 : 0, base.fo.forces, base.params ? 1 : 0};
-    auto it = g_tuned.find(key);
-    if (it != g_tuned.end()) {
-        *out = it->second;
-        return ASSIST_SUCCESS;
-    }
-    const int m = base.nsys < kTuneSample ? base.nsys : kTuneSample;
-    const size_t sw = (size_t)m * base.nvec * 6;
-    std::vector<double> h0(m), h1(m);
-    DevBuf<double> st, t1;
-    DevBuf<int> status;
-    if (!st.alloc(sw) || !t1.alloc(m) || !status.alloc(m)) return ASSIST_BATCH_ERROR_DEVICE;
-    if (!hip_ok(hipMemcpy(h0.data(), base.t0, m * sizeof(double), hipMemcpyDeviceToHost), "hipMemcpy") ||
-        !hip_ok(hipMemcpy(h1.data(), base.t1, m * sizeof(double), hipMemcpyDeviceToHost), "hipMemcpy"))
-        return ASSIST_BATCH_ERROR_DEVICE;
-    for (int i = 0; i < m; i++) {
-        const double d = h1[i] - h0[i];
-        h1[i] = h0[i] + (d > kTuneSpan ? kTuneSpan : (d < -kTuneSpan ? -kTuneSpan : d));
-    }
-    if (!hip_ok(hipMemcpy(t1.p, h1.data(), m * sizeof(double), hipMemcpyHostToDevice), "hipMemcpy"))
-        return ASSIST_BATCH_ERROR_DEVICE;
-    IntegrateArgs a = base;
-    a.nsys = m;
-    a.states = st.p;
-    a.t1 = t1.p;
-    a.status = status.p;
-    a.steps = a.evals = a.rejected = nullptr;
-    a.t_out = nullptr;
-    a.trace = nullptr;
-    a.trace_count = nullptr;
-    a.snap_in = nullptr;
-    a.snap_out = nullptr;
-    a.t_pause = nullptr;
-    a.archive = nullptr;
-    a.archive_count = nullptr;
-    a.archive_cap = 0;
-    LaunchShape one;
-    one.G = 1;
-    LaunchShape one_small = one;
-    one_small.threads = 128;
-    LaunchShape best;
-    float best_ms = 1e30f;
-    for (const LaunchShape& sh : {row_shape(m), one, one_small}) {
-        // each shape runs twice and keeps the faster time: a kernel's first launch can include loading
-        // its code, which the events around it would count
-        float ms = 1e30f;
-        for (int rep = 0; rep < 2; rep++) {
-            if (!hip_ok(hipMemcpyAsync(st.p, base.states, sw * sizeof(double), hipMemcpyDeviceToDevice, s),
-                        "hipMemcpyAsync"))
-                return ASSIST_BATCH_ERROR_DEVICE;
-            float t_ms = 0.f;
-            const int rc = run_ias15(a, mixed, sh, 0, s, &t_ms, nullptr, false, false);
-            if (rc) return rc;
-            if (t_ms < ms) ms = t_ms;
-        }
-        if (ms < best_ms) {
-            best_ms = ms;
-            best = sh;
-        }
-    }
-    g_tuned[key] = best;
-    *out = best;
     return ASSIST_SUCCESS;
 }
 
@@ -1082,10 +998,7 @@ static int integrate_device_locked(const struct assist_ephem* ephem, const struc
     // the substep cache pays when attempts take several passes: by default it is off with the
     // first-pass stop (configuration 4 mixed+learned: 158.3 ms without it, 161.9 ms with it)
     const bool cache = cfg.substep_cache_off < 0 || (cfg.substep_cache_off == 0 && a.io.pc_tol1 <= 0.0);
-    if (choose && nv == 1 && n >= kTuneMinSystems && !dense) {
-        rc = tuned_shape(a, mixed, s, &shape);
-        if (rc) return rc;
-    }
+    if (choose && nv == 1 && n >= kLaneMinSystems && !dense) shape = LaunchShape{1, kIas15Block, 1};
     // large batches: hand out the systems of highest expected cost first (longest spans, smallest
     // perihelia), so that the launch does not end on an expensive system handed out last
     if (n >= kOrderMinSystems && !dense && d_t1 && !a.snap_in) {

@@ -406,8 +406,10 @@ int assist_batch_integrate_device_ex(const struct assist_ephem* ephem, const str
  * routine: its scratch (the work-queue counter and the b/e records of at most 65 536 resident
  * lanes, 22 MB) is a static device array of the library, which every GPU the library runs on holds
  * until the process ends, and the grid is capped to it.  It runs without the substep cache, the
- * autotuner, the queue order, graph capture and timing (same results bit for bit; use_graph = 1
- * returns ASSIST_BATCH_ERROR_UNSUPPORTED).  The ephemeris must already be resident on the GPU
+ * queue order, graph capture and timing (use_graph = 1 returns ASSIST_BATCH_ERROR_UNSUPPORTED), on 16
+ * lanes per system unless cfg chooses others: the allocating entry point's results bit for bit, except
+ * for real-only batches of 131 072 systems or more, which that one runs on one lane per system (equal
+ * to round-off).  The ephemeris must already be resident on the GPU
  * (any other batched call with it makes it so; otherwise ASSIST_BATCH_ERROR_UNSUPPORTED).  Calls
  * that overlap on one GPU share that array and race: the library's lock serialises calls from
  * threads of one process, but not from several processes on one GPU.  Returns after the kernel
