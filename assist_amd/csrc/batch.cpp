@@ -551,22 +551,26 @@ constexpr int kOrderMinSystems = 16384;
 // times as long as blocks of 256 at every size.)
 constexpr int kLaneMinSystems = 131072;
 
-// The shape of the 16-lane kernel for n systems.  A trip of a wave takes as long with one system as
-// with four, so systems go one to a wave while every SIMD has room for another wave (blocks of one
-// wave, which spread over the CUs), then up to four to a wave (one block of four waves per CU), and
-// only then does a second wave per SIMD pay (blocks of three waves, two per CU, all that the
-// ephemeris tables in LDS leave room for): 4,096 systems x 7 vectors over 3,650 days take 37.4 ms with
-// one wave per SIMD and 45.0 ms with blocks of three waves, 262,144 over 365 days 152 against 118.7 ms.
-LaunchShape row_shape(int n) {
+// The shape of the 16-lane kernel.  A trip of a wave takes as long with one system as with four, so
+// systems go one to a wave while every SIMD has room for another wave (blocks of one wave, which spread
+// over the CUs), then up to four to a wave (one block of four waves per CU), and only then does a second
+// wave per SIMD pay, where the kernel's registers allow it (blocks of three waves, two per CU, all that
+// the ephemeris tables in LDS leave room for).  The FP64 kernels with partials and Marsden parameters, or
+// with other forces than the default ones, hold one wave per SIMD: a CU takes one block of them, and one
+// of three waves would leave its fourth SIMD without work.  Blocks of four waves and of three (ms): 4,096
+// systems x 7 vectors over 3,650 d 38.0 and 45.9; 262,144 x 7 over 365 d 287 and 230, in the mixed form
+// from the learned start 139 and 107; with one wave per SIMD, 20,011 x 8 with Marsden models over 300 d
+// 22.0 and 28.8, 65,536 x 8 over 100 d 32.3 and 43.0.
+LaunchShape row_shape(const IntegrateArgs& a, bool mixed) {
     int dev = 0, ncu = 0;
     if (hipGetDevice(&dev) != hipSuccess ||
         hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess)
         ncu = 256;
     LaunchShape sh;
     sh.G = kRowLanes;
-    sh.waves = 1;
+    sh.waves = ias15_row_waves(a, mixed);
     const long long simds = 4LL * ncu;
-    sh.threads = n <= simds ? 64 : (n <= 4 * simds ? 256 : 192);
+    sh.threads = a.nsys <= simds ? 64 : (a.nsys <= 4 * simds || sh.waves == 1 ? 256 : 192);
     return sh;
 }
 
@@ -994,7 +998,7 @@ static int integrate_device_locked(const struct assist_ephem* ephem, const struc
     // with no launch override: 16 lanes per system, or one (the checkpoint features and the extended
     // force model run on the group kernels alone, on 8 lanes or, below, on one)
     const bool choose = lanes_req == 0 && cfg.block_size == 0 && cfg.waves_per_simd == 0 && !ext && !ias15_snap(a);
-    if (choose) shape = row_shape(n);
+    if (choose) shape = row_shape(a, mixed);
     // the substep cache pays when attempts take several passes: by default it is off with the
     // first-pass stop (configuration 4 mixed+learned: 158.3 ms without it, 161.9 ms with it)
     const bool cache = cfg.substep_cache_off < 0 || (cfg.substep_cache_off == 0 && a.io.pc_tol1 <= 0.0);
@@ -1066,18 +1070,6 @@ int assist_batch_integrate_device_noalloc(const struct assist_ephem* ephem, cons
     const bool mixed = cfg.precision == ASSIST_PRECISION_MIXED;
     const bool ext = ext_model(a.fo);
     if (ext && mixed) return ASSIST_BATCH_ERROR_UNSUPPORTED;
-    LaunchShape shape;
-    if (cfg.lanes_per_system == 0 && cfg.block_size == 0 && cfg.waves_per_simd == 0 && !ext) {
-        shape = row_shape(n);
-    } else {
-        shape.G = lanes_for(nv, cfg.lanes_per_system);
-        shape.threads = cfg.block_size > 0 ? cfg.block_size : kIas15Block;
-        shape.waves = 1;
-        if (shape.G < 0 || shape.threads % 64 != 0 || shape.threads > kIas15Block || shape.threads % shape.G != 0)
-            return ASSIST_BATCH_ERROR_ARG;
-        if (cfg.waves_per_simd != 0 && cfg.waves_per_simd != 1) return ASSIST_BATCH_ERROR_UNSUPPORTED;
-    }
-    const int G = shape.G, threads = shape.threads;
     a.io.epsilon = cfg.epsilon;
     a.io.min_dt = cfg.min_dt;
     a.io.dt_initial = cfg.dt_initial;
@@ -1094,6 +1086,18 @@ int assist_batch_integrate_device_noalloc(const struct assist_ephem* ephem, cons
     a.status = d_status;
     a.steps = d_steps;
     a.evals = d_evals;
+    LaunchShape shape;
+    if (cfg.lanes_per_system == 0 && cfg.block_size == 0 && cfg.waves_per_simd == 0 && !ext) {
+        shape = row_shape(a, mixed);
+    } else {
+        shape.G = lanes_for(nv, cfg.lanes_per_system);
+        shape.threads = cfg.block_size > 0 ? cfg.block_size : kIas15Block;
+        shape.waves = 1;
+        if (shape.G < 0 || shape.threads % 64 != 0 || shape.threads > kIas15Block || shape.threads % shape.G != 0)
+            return ASSIST_BATCH_ERROR_ARG;
+        if (cfg.waves_per_simd != 0 && cfg.waves_per_simd != 1) return ASSIST_BATCH_ERROR_UNSUPPORTED;
+    }
+    const int G = shape.G, threads = shape.threads;
     std::lock_guard<std::mutex> lock(g_launch_mutex);
     double* scr = nullptr;
     int dev = 0, ncu = 0, per_cu = 0;

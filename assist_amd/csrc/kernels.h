@@ -152,6 +152,8 @@ hipError_t launch_ias15_row(const IntegrateArgs& a, bool mixed, int blocks, int 
 hipError_t launch_ias15_row_late(const IntegrateArgs& a, bool mixed, int blocks, int threads, hipStream_t s,
                                  bool set_attributes = true);
 hipError_t ias15_row_occupancy(const IntegrateArgs& a, bool mixed, int threads, int* blocks_per_cu, bool late = false);
+// Waves per SIMD that the 16-lane kernel of a launch is compiled for (its registers hold no more).
+int ias15_row_waves(const IntegrateArgs& a, bool mixed);
 size_t ias15_row_lds_bytes(int threads);
 // The one-lane kernel of real-only launches (lane_kernel.hip), without checkpoint features, dense output
 // or the extended force model; its scratch is 42 doubles per launched thread.

@@ -937,16 +937,23 @@ static const void* row_fn(int model) {
                                   : (const void*)ias15_row_kernel<M, NV, J, kModelAny, Late>;
 }
 
-static const void* row_lookup(const IntegrateArgs& a, bool mixed, bool late = false) {
+// The force model that a launch's kernel is compiled for.
+static int row_model(const IntegrateArgs& a, bool mixed) {
     const bool std_forces = a.fo.forces == kStdForces && a.fo.gr_eih_sources > 0;
-    int m = kModelAny;
-    if (mixed || std_forces) m = !a.params ? kModelGravity : (mixed ? kModelAny : kModelStd);
+    if (!mixed && !std_forces) return kModelAny;
+    return !a.params ? kModelGravity : (mixed ? kModelAny : kModelStd);
+}
+
+static const void* row_lookup(const IntegrateArgs& a, bool mixed, bool late = false) {
+    const int m = row_model(a, mixed);
     if (late) return a.nvec != 1 ? nullptr : (mixed ? row_fn<true, 1, false, true>(m) : row_fn<false, 1, false, true>(m));
     if (a.nvec == 1) return mixed ? row_fn<true, 1, false>(m) : row_fn<false, 1, false>(m);
     if (a.nvec <= 4) return mixed ? row_fn<true, 1, true>(m) : row_fn<false, 1, true>(m);
     if (a.nvec <= 8) return mixed ? row_fn<true, 2, true>(m) : row_fn<false, 2, true>(m);
     return nullptr;
 }
+
+int ias15_row_waves(const IntegrateArgs& a, bool mixed) { return row_waves(mixed, a.nvec > 1, row_model(a, mixed)); }
 
 size_t ias15_row_lds_bytes(int threads) {
     return (kTabWords + (size_t)(threads / 64) * kRowWaveWords) * sizeof(double);

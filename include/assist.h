@@ -302,7 +302,8 @@ struct assist_batch_stats {
                                           the entry points on device buffers leave them 0 (their
                                           per-system counts are in d_steps / d_evals) */
     double kernel_ms;     /* device time of the integration kernel (HIP events) */
-    int lanes_per_system, block_size, grid_blocks, waves_per_simd;
+    int lanes_per_system, block_size, grid_blocks;
+    int waves_per_simd;   /* 1 or 2: the register budget of the kernel that ran */
 };
 
 void assist_batch_config_default(struct assist_batch_config* cfg);
