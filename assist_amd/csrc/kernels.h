@@ -145,7 +145,9 @@ hipError_t launch_ias15(const IntegrateArgs& a, int G, bool mixed, int waves, in
 hipError_t ias15_occupancy(int G, bool mixed, int waves, bool ext, bool snap, int nvec, int threads,
                            int* blocks_per_cu);
 // The 16-lane kernel (row_kernel.hip), for launches without checkpoint features or the extended
-// force model; its scratch is 28 doubles per launched thread at most.
+// force model; its scratch is row_scratch_words(nvec) doubles per launched thread (the b and e of one
+// component of one or two vectors).
+__host__ __device__ constexpr int row_scratch_words(int nvec) { return nvec <= 4 ? 14 : 28; }
 hipError_t launch_ias15_row(const IntegrateArgs& a, bool mixed, int blocks, int threads, hipStream_t s,
                             bool set_attributes = true);
 // The same for the systems of a.late (its queue starts at the grid's rows).
@@ -168,10 +170,14 @@ inline bool ext_model(const ForceOpts& f) { return f.geocentric != 0 || ((f.forc
 size_t ias15_lds_bytes(int G, int nvec, int threads, int waves, bool ext);
 hipError_t launch_set_counter(int* q, int v, hipStream_t s);
 // Scratch of the allocation-free entry point: a static device array of the library (22 MB per
-// GPU): kNoAllocHeadWords doubles for the work-queue counter, then the b/e records of up to
-// kNoAllocLanes resident lanes (42 doubles each).  *ptr receives its device address on the
+// GPU): kNoAllocHeadWords doubles for the work-queue counter, then kNoAllocLanes x 42 for the b/e records
+// of the resident lanes: kNoAllocLanes of the group and one-lane kernels (42 doubles each), more of the
+// 16-lane kernel (noalloc_lanes).  *ptr receives its device address on the
 // current device (looked up once per device).
 constexpr int kNoAllocLanes = 65536;
+inline long long noalloc_lanes(int G, int nvec) {
+    return G == kRowLanes ? (long long)kNoAllocLanes * 42 / row_scratch_words(nvec) : kNoAllocLanes;
+}
 constexpr int kNoAllocHeadWords = 32;
 constexpr int kNoAllocMaxDevices = 64;
 hipError_t noalloc_scratch(double** ptr);

@@ -948,6 +948,7 @@ static const void* row_lookup(const IntegrateArgs& a, bool mixed, bool late = fa
     const int m = row_model(a, mixed);
     if (late) return a.nvec != 1 ? nullptr : (mixed ? row_fn<true, 1, false, true>(m) : row_fn<false, 1, false, true>(m));
     if (a.nvec == 1) return mixed ? row_fn<true, 1, false>(m) : row_fn<false, 1, false>(m);
+    static_assert(row_scratch_words(4) == 14 * 1 && row_scratch_words(8) == 14 * 2, "14 words per component and vector");
     if (a.nvec <= 4) return mixed ? row_fn<true, 1, true>(m) : row_fn<false, 1, true>(m);
     if (a.nvec <= 8) return mixed ? row_fn<true, 2, true>(m) : row_fn<false, 2, true>(m);
     return nullptr;

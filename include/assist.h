@@ -404,8 +404,8 @@ int assist_batch_integrate_device_ex(const struct assist_ephem* ephem, const str
 /* Allocation-free variant of assist_batch_integrate_device (no counterpart in the reference):
  * for callers that cannot allocate device memory -- code under HIP graph capture, tight serving
  * loops, harnesses that forbid hipMalloc.  It calls no hipMalloc, hipFree or other allocating
- * routine: its scratch (the work-queue counter and the b/e records of at most 65 536 resident
- * lanes, 22 MB) is a static device array of the library, which every GPU the library runs on holds
+ * routine: its scratch (the work-queue counter and 22 MB for the b/e records of the resident
+ * lanes: 65 536, or up to 196 608 on 16 lanes per system) is a static device array of the library, which every GPU the library runs on holds
  * until the process ends, and the grid is capped to it.  It runs without the substep cache, the
  * queue order, graph capture and timing (use_graph = 1 returns ASSIST_BATCH_ERROR_UNSUPPORTED), on 16
  * lanes per system unless cfg chooses others: the allocating entry point's results bit for bit, except
