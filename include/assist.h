@@ -379,7 +379,13 @@ struct assist_batch_extra {
      * the config sets them.  Not with dense output (ASSIST_BATCH_ERROR_UNSUPPORTED).
      * snapshot_out: each system's snapshot when it stops (finished, paused or failed).
      * t_pause: system i stops with status ASSIST_SYSTEM_PAUSED at the first step boundary at or
-     * past t_pause[i] in its direction (unless that boundary is t1). */
+     * past t_pause[i] in its direction (unless that boundary is t1).
+     * A resumed run takes the steps of an uninterrupted one: bit for bit those of an uninterrupted
+     * run with snapshot_out on the same lanes per system, and those of a plain launch on 2, 4, 8 or
+     * 16 lanes (8 and 16 are equal) in FP64 and of the real particle in the mixed form (whose FP32
+     * partials round differently in a few variational vectors, by units in the last place).  A plain
+     * launch on one lane (lanes_per_system = 1, or 131 072 real particles and more) sums in another
+     * order and agrees to round-off. */
     const double* snapshot_in;
     double* snapshot_out;
     const double* t_pause;
