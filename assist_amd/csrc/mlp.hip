@@ -306,7 +306,7 @@ __global__ void __launch_bounds__(64 * kTWaves) mlp_train_kernel(TrainArgs args)
     float db1[kTNt] = {}, db2[kTNt] = {}, db3[kTNt] = {}, db4 = 0.f, loss = 0.f;
     TrainArgs g = args;
     for (int base = blockIdx.x * kTRows; base < args.M; base += gridDim.x * kTRows) {
-        // (opaque per trip: the weight fragments are the same for every 64 rows, and hoisted out of
+        // (opaque per trip: the weight fragments are the same for every 32 rows, and hoisted out of
         // the loop they would not fit the registers)
         int zero = 0;
         asm volatile("" : "+s"(zero));
@@ -428,7 +428,7 @@ __global__ void __launch_bounds__(64 * kTWaves) mlp_train_kernel(TrainArgs args)
 #pragma unroll
         for (int nt = 0; nt < 2; nt++) out[kOff4 + in * kOut + nt * 16 + r] = gw4[nt][j];
     }
-    // bias gradients: over a tile's rows by lane exchange, over the four tiles through LDS
+    // bias gradients: over a tile's rows by lane exchange, over the two tiles through LDS
     float* const s_db = (float*)s_inT;  // [kTRows / 16][kTBias]
     auto put_bias = [&](float v, int at) {
         v += __shfl_xor(v, 16, 64);
@@ -461,7 +461,7 @@ __global__ void __launch_bounds__(64 * kTWaves) mlp_train_kernel(TrainArgs args)
 
 // Gradients and loss from the workgroups' sums: 64 groups of four parameters per block, each
 // summed by four waves that take every fourth workgroup's slice (the slices stream from L2; one
-// thread per group alone would leave the loads of 128 slices in a chain).
+// thread per group alone would leave the loads of up to 256 slices in a chain).
 __global__ void __launch_bounds__(256) reduce_grad_kernel(const float* __restrict__ part, int nblocks, int M, float* grad,
                                                           float* loss) {
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
@@ -497,7 +497,6 @@ size_t w_off(int l) {
     for (int i = 0; i < l; i++) o += (size_t)kDims[i] * kDims[i + 1] + kDims[i + 1];
     return o;
 }
-size_t b_off(int l) { return w_off(l) + (size_t)kDims[l] * kDims[l + 1]; }
 
 bool ok(hipError_t e, const char* what) {
     if (e == hipSuccess) return true;
