@@ -370,6 +370,7 @@ struct Workspace {
     double* scratch = nullptr;
     size_t scratch_words = 0;
     int* queue = nullptr;  // the work queue's counter, then the number of late systems
+    double* expected = nullptr;  // steps expected of a batch, and of its costliest system
     double* late = nullptr;
     size_t late_cap = 0;
     hipEvent_t ev0 = nullptr, ev1 = nullptr, ev_in = nullptr;
@@ -402,7 +403,9 @@ int ensure_workspace(size_t scratch_words) {
         g_ws.graphs.clear();  // (those of another device are not destroyed from this one)
         g_ws = Workspace();
         g_ws.device = dev;
-        if (!hip_ok(hipMalloc(&g_ws.queue, 2 * sizeof(int)), "hipMalloc(queue)")) return ASSIST_BATCH_ERROR_DEVICE;
+        if (!hip_ok(hipMalloc(&g_ws.queue, 2 * sizeof(int)), "hipMalloc(queue)") ||
+            !hip_ok(hipMalloc(&g_ws.expected, 2 * sizeof(double)), "hipMalloc(expected)"))
+            return ASSIST_BATCH_ERROR_DEVICE;
         if (!hip_ok(hipEventCreate(&g_ws.ev0), "hipEventCreate") || !hip_ok(hipEventCreate(&g_ws.ev1), "hipEventCreate") ||
             !hip_ok(hipEventCreateWithFlags(&g_ws.ev_in, hipEventDisableTiming), "hipEventCreate") ||
             !hip_ok(hipStreamCreateWithFlags(&g_ws.graph_stream, hipStreamNonBlocking), "hipStreamCreate"))
@@ -539,17 +542,22 @@ struct LaunchShape {
 
 // Batches of this size or more hand out their systems in the queue order.
 constexpr int kOrderMinSystems = 16384;
-// Real-only batches of this size or more take one lane per system, everything else 16.  The line is a
-// number of systems alone: the two kernels sum in another order, and results must not depend on which of
-// them a timing prefers.  One lane per system needs 65,536 systems to give every SIMD one wave; its last
-// systems run on 16 lanes (lane_kernel.hip).  On one lane and on 16 (ms, mixed form): 65,536 systems over
-// 365 d 15.9 and 18.1, over 40 d 4.8 and 3.9, over uneven spans up to 10,000 d 188 and 150.  In double
-// precision and in the mixed form: 131,072 over 1 d 4.4 and 8.9, 4.6 and 8.3; over 40 d 12.0 and 16.5, 9.0
-// and 13.1; over 365 d 49.6 and 63.4, 26.9 and 41.4; over uneven spans from 30 to 3,000 d 143 and 112, 75
-// and 67; 262,144 over those 218 and 208, 107 and 133; over 365 d 87 and 126, 44 and 82; 1,048,576 over
-// 365 d 333 and 498, 165 and 325.  (Blocks of 128 threads, of which a CU's LDS holds one, took 1.2 to 1.9
-// times as long as blocks of 256 at every size.)
+// Launches without overrides take 16 lanes per system, or, real particles alone, one.  The choice follows
+// from the batch, not from a timing: the two kernels sum in another order, and results must not depend on
+// which of them a timing prefers.  One lane per system needs 65,536 systems to give every SIMD one wave; its
+// last systems run on 16 lanes (lane_kernel.hip).  It pays from kLaneMinSystems on.  On one lane and on 16
+// (ms, mixed form): 65,536 systems over 365 d 15.9 and 18.1, over 40 d 4.8 and 3.9; in double precision and
+// in the mixed form: 131,072 over 1 d 4.4 and 8.9, 4.6 and 8.3; over 40 d 12.0 and 16.5, 9.0 and 13.1; over
+// 365 d 49.6 and 63.4, 26.9 and 41.4; 1,048,576 over 365 d 333 and 498, 165 and 325.  (Blocks of 128
+// threads, of which a CU's LDS holds one, took 1.2 to 1.9 times as long as blocks of 256 at every size.)
 constexpr int kLaneMinSystems = 131072;
+// An uneven batch ends on its costliest systems, which a lane integrates more slowly than 16 do: one lane
+// pays where the steps that all systems take (expected_share) are at least kLaneShare times the costliest
+// system's.  Spans from 30 to 3,000 d, on one lane and on 16 (ms, double precision; mixed form), at that
+// ratio: 11,400 (131,072 systems) 142 and 111, 74 and 67; 15,500 (150,001) 148 and 119, 83 and 81; 16,100
+// (200,003) 177 and 159, 94 and 102; 20,000 (262,144) 219 and 208, 106 and 133; 33,000 (131,072 over 365 d)
+// above.  (The line is the mixed form's.)
+constexpr double kLaneShare = 15000.0;
 
 // The shape of the 16-lane kernel.  A trip of a wave takes as long with one system as with four, so
 // systems go one to a wave while every SIMD has room for another wave (blocks of one wave, which spread
@@ -588,33 +596,21 @@ int group_block(int n, int G) {
 // Checkpoint, pause and archive launches of real particles run on ias15_kernel, on 8 lanes per system or on
 // one.  One lane does about a third of the work per evaluation, but its launch lasts as long as its costliest
 // system, which a lane integrates 2.5 times slower than 8 lanes do: it wins where the batch keeps 65,536
-// lanes busy for longer than that.  With the steps that a system takes (about 7 + 0.15 |t1 - t0| / q, the
-// fit behind the queue order) the line is sum of the steps = kOneLaneShare x the costliest system's.
-// Eight lanes' time over one lane's, in double precision and in the mixed form, at that share: 26,000
-// (131,072 systems, spans from 30 to 365 d) 0.69, 0.92; 33,000 (131,072 over 365 d) 0.90, 1.14; 39,000
-// (180,001, 30 to 365 d) 0.80, 1.24; 44,000 (262,144, 30 to 365 d) 1.17, 1.30; 45,000 (180,001 over 365 d)
-// 1.30, 1.73; 106,000 (131,072 over 5 d) 2.5, 2.7; 262,000 (1,048,576 over 365 d) 2.0, 2.4.
-constexpr double kOneLaneShare = 42000.0;
-constexpr int kShareSample = 1024;  // systems of the sorted queue that stand for all
+// lanes busy for longer than that.  Eight lanes' time over one lane's, in double precision and in the mixed
+// form, at the ratio of all systems' steps to the costliest one's: 26,000 (131,072 systems, spans from 30 to
+// 365 d) 0.69, 0.92; 33,000 (131,072 over 365 d) 0.90, 1.14; 39,000 (180,001, 30 to 365 d) 0.80, 1.24; 44,000
+// (262,144, 30 to 365 d) 1.17, 1.30; 45,000 (180,001 over 365 d) 1.30, 1.73; 106,000 (131,072 over 5 d) 2.5,
+// 2.7; 262,000 (1,048,576 over 365 d) 2.0, 2.4.
+constexpr double kGroupLaneShare = 42000.0;
 
-// Whether the batch's n sorted queue keys (device; launch_span_order) put it on one lane.
-int one_lane_share(const unsigned long long* keys, int n, hipStream_t s, bool* one) {
-    const int m = std::min(n, kShareSample);
-    const size_t stride = (size_t)(n / m) * sizeof *keys;
-    unsigned long long h[kShareSample];
-    if (!hip_ok(hipMemcpy2DAsync(h, sizeof *h, keys, stride, sizeof *h, (size_t)m, hipMemcpyDeviceToHost, s), "hipMemcpy2DAsync") ||
-        !hip_ok(hipStreamSynchronize(s), "queue order"))
+// Steps that a batch takes in all over those of its costliest system, from its n sorted queue keys (device).
+int expected_share(const unsigned long long* keys, int n, hipStream_t s, double* share) {
+    double h[2];
+    if (!hip_ok(launch_expected_steps(keys, n, g_ws.expected, s), "launch(expected steps)") ||
+        !hip_ok(hipMemcpyAsync(h, g_ws.expected, sizeof h, hipMemcpyDeviceToHost, s), "hipMemcpyAsync") ||
+        !hip_ok(hipStreamSynchronize(s), "expected steps"))
         return ASSIST_BATCH_ERROR_DEVICE;
-    double sum = 0.0, most = 0.0;
-    for (int i = 0; i < m; i++) {
-        const unsigned long long bits = h[i] & ~kKeyRateMask;
-        double span;
-        memcpy(&span, &bits, sizeof span);
-        const double steps = 7.0 + 0.15e-3 * span * (double)(h[i] & kKeyRateMask);
-        sum += steps;
-        most = std::max(most, steps);
-    }
-    *one = sum < 1e300 && (double)n / m * sum >= kOneLaneShare * most;
+    *share = h[0] < 1e300 ? h[0] / h[1] : 0.0;  // (0 where a span is infinite)
     return ASSIST_SUCCESS;
 }
 
@@ -1002,7 +998,6 @@ static int integrate_device_locked(const struct assist_ephem* ephem, const struc
     // the substep cache pays when attempts take several passes: by default it is off with the
     // first-pass stop (configuration 4 mixed+learned: 158.3 ms without it, 161.9 ms with it)
     const bool cache = cfg.substep_cache_off < 0 || (cfg.substep_cache_off == 0 && a.io.pc_tol1 <= 0.0);
-    if (choose && nv == 1 && n >= kLaneMinSystems && !dense) shape = LaunchShape{1, kIas15Block, 1};
     // large batches: hand out the systems of highest expected cost first (longest spans, smallest
     // perihelia), so that the launch does not end on an expensive system handed out last
     if (n >= kOrderMinSystems && !dense && d_t1 && !a.snap_in) {
@@ -1015,15 +1010,13 @@ static int integrate_device_locked(const struct assist_ephem* ephem, const struc
                     "launch(queue order)"))
             return ASSIST_BATCH_ERROR_DEVICE;
         a.order = g_ws.order;
-        // (a resumed batch keeps its snapshots' lanes)
-        if (ias15_snap(a) && nv == 1 && lanes_req == 0 && cfg.block_size == 0 && cfg.waves_per_simd == 0 && !ext) {
-            bool one = false;
-            rc = one_lane_share(g_ws.okeys_alt, n, s, &one);
+        // (checkpoint launches: a resumed batch keeps its snapshots' lanes)
+        const bool group = ias15_snap(a) && lanes_req == 0 && cfg.block_size == 0 && cfg.waves_per_simd == 0 && !ext;
+        if (nv == 1 && (group || (choose && n >= kLaneMinSystems))) {
+            double share = 0.0;
+            rc = expected_share(g_ws.okeys_alt, n, s, &share);
             if (rc) return rc;
-            if (one) {
-                shape.G = 1;
-                shape.threads = group_block(n, 1);
-            }
+            if (share >= (group ? kGroupLaneShare : kLaneShare)) shape = LaunchShape{1, group_block(n, 1), 1};
         }
     }
     float ms = 0.f;

@@ -191,6 +191,9 @@ size_t span_order_temp_bytes(int n);
 hipError_t launch_span_order(const DevEphem* E, int n, int nvec, const double* t0, const double* t1,
                              const double* states, unsigned long long* keys, unsigned long long* keys_alt, int* vals,
                              int* order, void* temp, size_t temp_bytes, hipStream_t s);
+// From the sorted keys: out[0] the steps that the batch is expected to take in all, out[1] those of its
+// costliest system, from a sample of the queue (no numbers where a span is infinite).
+hipError_t launch_expected_steps(const unsigned long long* keys, int n, double* out, hipStream_t s);
 // States at query times from step archives (IntegrateArgs::archive layout): query q asks for
 // system qsys[q] (0 <= qsys[q] < nsys, else status kBadSystem) at qt[q]; out[q][nvec][6];
 // status kCoverage outside the archived steps.

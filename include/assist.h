@@ -384,7 +384,8 @@ struct assist_batch_extra {
      * run with snapshot_out on the same lanes per system, and those of a plain launch on 2, 4, 8 or
      * 16 lanes (8 and 16 are equal) in FP64 and of the real particle in the mixed form (whose FP32
      * partials round differently in a few variational vectors, by units in the last place).  A plain
-     * launch on one lane (lanes_per_system = 1, or 131 072 real particles and more) sums in another
+     * launch on one lane (lanes_per_system = 1, or most batches of 131 072 real particles
+     * and more) sums in another
      * order and agrees to round-off. */
     const double* snapshot_in;
     double* snapshot_out;
@@ -415,8 +416,8 @@ int assist_batch_integrate_device_ex(const struct assist_ephem* ephem, const str
  * until the process ends, and the grid is capped to it.  It runs without the substep cache, the
  * queue order, graph capture and timing (use_graph = 1 returns ASSIST_BATCH_ERROR_UNSUPPORTED), on 16
  * lanes per system unless cfg chooses others: the allocating entry point's results bit for bit, except
- * for real-only batches of 131 072 systems or more, which that one runs on one lane per system (equal
- * to round-off).  The ephemeris must already be resident on the GPU
+ * for real-only batches of 131 072 systems or more, which that one runs on one lane per system unless
+ * their spans are very uneven (equal to round-off).  The ephemeris must already be resident on the GPU
  * (any other batched call with it makes it so; otherwise ASSIST_BATCH_ERROR_UNSUPPORTED).  Calls
  * that overlap on one GPU share that array and race: the library's lock serialises calls from
  * threads of one process, but not from several processes on one GPU.  Returns after the kernel

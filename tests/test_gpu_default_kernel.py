@@ -1,5 +1,6 @@
-"""The kernel that a launch without overrides takes follows from the batch alone: real-only batches of
-131,072 systems or more run on one lane per system, whatever ran before them in the process.  Main-belt
+"""The kernel that a launch without overrides takes follows from the batch alone, whatever ran before it in
+the process: real-only batches of 131,072 systems or more run on one lane per system, unless their spans are
+so uneven that the launch would end on a few costly ones.  Main-belt
 orbits over at most 20 days, on which the kernels differ by round-off alone: steps of days, each leaving a
 few units in the last place of 3 au (1e-4 m each), so 1 cm holds many of them, and a wrong record, body or
 hand-over moves a position by kilometres."""
@@ -42,6 +43,24 @@ def test_default_choice_does_not_depend_on_earlier_calls(gpu, ephem, belt, preci
     assert (groups.status == 0).all()
     d = np.linalg.norm(auto.states[:, 0, :3] - groups.states[:, 0, :3], axis=-1) * AU_M
     assert d.max() <= (0.01 if precision == 0 else 1.0)
+
+
+@pytest.mark.parametrize("precision", [0, 1])
+def test_uneven_spans_take_16_lanes(gpu, ephem, belt, precision):
+    """One span in a hundred is 100 days, the others half a day: all steps together are 50,000 times the
+    costliest system's (one lane); with 3,000 days, 3,400 times.  On 16 lanes the bits are the 8-lane
+    kernel's."""
+    from assist_amd import batch
+    for long, lanes in ((100.0, 1), (3000.0, 16)):
+        t1 = np.full(N, 0.5)
+        t1[::100] = -long
+        r = batch.integrate(ephem, 0.0, t1, belt, config=batch.BatchConfig.default(precision=precision))
+        assert r.stats.lanes_per_system == lanes and (r.status == 0).all()
+        if lanes == 16:
+            groups = batch.integrate(ephem, 0.0, t1, belt,
+                                     config=batch.BatchConfig.default(precision=precision, lanes_per_system=8))
+            np.testing.assert_array_equal(r.states, groups.states)
+            np.testing.assert_array_equal(r.steps, groups.steps)
 
 
 def test_below_the_line_16_lanes(gpu, ephem, belt):
