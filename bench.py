@@ -229,9 +229,15 @@ def copy_calibration(mib):
     dst.free()
 
 
-def measured_traffic(config, form, n):
+def kernel_name(lanes, waves):
+    """The integration kernel that a launch of the stats' lanes per system runs here (real particles alone
+    on one lane; no checkpoint features)."""
+    return {16: "ias15_row_kernel", 1: "ias15_lane_kernel" if waves == 1 else "ias15_kernel"}.get(lanes, "ias15_kernel")
+
+
+def measured_traffic(config, form, n, kernel):
     """HBM bytes per launch of the integration kernel from the committed counter profile
-    (profiles/ias15_kernel_traffic.md), or None when this workload and form were not profiled."""
+    (profiles/ias15_kernel_traffic.md), or None when this workload, form and kernel were not profiled."""
     path = os.path.join(ROOT, "profiles", "ias15_kernel_traffic.md")
     try:
         txt = open(path).read()
@@ -240,7 +246,7 @@ def measured_traffic(config, form, n):
     for line in txt.splitlines():
         if line.startswith("traffic_json:"):
             for row in json.loads(line.split(":", 1)[1]):
-                if row["config"] == config and row["form"] == form and row["systems"] == n:
+                if (row["config"], row["form"], row["systems"], row["kernel"]) == (config, form, n, kernel):
                     return row["bytes_per_launch"]
     return None
 
@@ -360,7 +366,8 @@ def main():
     ach64 = f64 / (kms * 1e-3) / 1e12
     ach32 = f32 / (kms * 1e-3) / 1e12
     frac = ach64 / FP64_PEAK_TFLOPS + ach32 / FP32_PEAK_TFLOPS
-    traffic = measured_traffic(args.config, args.form, n)
+    kernel = kernel_name(st.lanes_per_system, st.waves_per_simd)
+    traffic = measured_traffic(args.config, args.form, n, kernel)
     dpos = np.linalg.norm(main_res["states"][:, 0, :3] - plain["states"][:, 0, :3], axis=-1) * 149597870700.0
     result = {
         "metric": "particle-days/sec (plain FP64 vs mixed+learned) at <=1 m 10-yr position error",
@@ -386,8 +393,8 @@ def main():
                      "frac": frac, "traffic": traffic,
                      "traffic_source": None if traffic is None else
                      "committed counter profile profiles/ias15_kernel_traffic.md (rocprofv3 --pmc FETCH_SIZE, "
-                     "WRITE_SIZE of this workload and form, scaled by a copy kernel), not measured in this run",
-                     "kernel": "ias15_kernel", "kernel_ms": kms, "flops_fp64_per_launch": f64,
+                     "WRITE_SIZE of this workload, form and kernel, scaled by a copy kernel), not measured in this run",
+                     "kernel": kernel, "kernel_ms": kms, "flops_fp64_per_launch": f64,
                      "flops_fp32_per_launch": f32, "achieved_fp64": ach64, "achieved_fp32": ach32,
                      "hbm_gbs": None if traffic is None else traffic / (kms * 1e-3) / 1e9},
         "integration": {"steps_total": int(main_res["steps"].sum()), "evals_total": int(main_res["evals"].sum()),
