@@ -25,7 +25,7 @@
 // wave.  Two waves per SIMD overlap theirs, and the ephemeris tables leave LDS for six waves per CU.
 // Measured on an MI355X against the 8-lane kernel: one system, FP64, 1.95 us per evaluation (4.67)
 // alone and 3.3 us (5.5) with 6 vectors; 4,096 x 7 vectors over 3,650 d 37 ms (61); 262,144 x 7 over
-// 365 d in the mixed form 104 ms (143); 65,536 uneven real-only spans up to 10,000 d 152 ms (297).
+// 365 d in the mixed form 107 ms (143); 65,536 uneven real-only spans up to 10,000 d 152 ms (297).
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
